@@ -508,66 +508,98 @@ __global__ void k_wind_c2e(const Solve *solves, int s) {
 }
 
 // Time-averaged winds of the current step from the FP64 basis (src/averaged_velocity.py:14-62).
-// u(t) = sum_m s_m(t) W_m; RK1: u_avg = u(t_{n-1}); RK2: upwind-interpolated extrapolation.
-// Writes dtype uavg / usgn on x-edges e in [i0-1, iend+1] (all rows) and likewise for v.
-template <typename T>
-__global__ void k_wind_avg(Solve *solves, int all) {
-  Solve &S = solves[blockIdx.z];
+// u(t) = sum_m s_m(t) W_m; RK1: u_avg = u(t_{n-1}); RK2: the upwind interpolation of the
+// extrapolated wind 1.5 u(t_{n-1}) - 0.5 u(t_{n-2}), whose basis coefficients are combined once
+// per thread (scalars), so an edge reads its basis values and those of its upwind neighbour, each
+// once.  Writes dtype uavg / usgn on x-edges e in [i0, iend] (all rows) and likewise for v.
+// Bound by memory latency: kWindEdges edges per thread over a flat index (no idle threads where
+// the edges of a row do not fill a block), every value of one stage requested before the first
+// is used.  With one block per row and a loop over the basis per value, RK2 with four fields took
+// 28 us per step at N = 256 FP64.
+// KB: basis fields, a compile-time count (1, or 4 as vf = 2 has) or 0 for any other.
+constexpr int kMaxBasis = 8;
+template <int KB>
+__device__ __forceinline__ double wind_comb(const double *W, int64_t bs, const double *s, int K) {
+  if constexpr (KB == 1) {
+    return wind_of_basis(s[0], W[0]);   // the same bits as the step's own (WIND)
+  } else {
+    double acc = 0.0;
+#pragma unroll
+    for (int m = 0; m < (KB ? KB : kMaxBasis); ++m)
+      if (m < K) acc += s[m] * W[m * bs];
+    return acc;
+  }
+}
+
+// Block blk of the x-edges (dir 0) or y-edges (dir 1) of panel p.
+template <typename T, int KB>
+__device__ __forceinline__ void wind_edges(const Solve &S, int p, int dir, int blk) {
   const csadv_solve_desc &D = S.d;
-  const int N = D.N, M = S.M, ld = D.ld, ldu = D.ldu, K = D.nbasis;
-  const int p = blockIdx.y;
-  const int i0 = NG, iend = N + NG;
-  if (!all && !D.unsteady) return;                                  // steady: set at init
-  if ((D.stop > 0 && D.ctl[1] >= D.stop) || D.ctl[0]) return;       // solve finished or halted
+  const int N = D.N, M = S.M, ld = D.ld, ldu = D.ldu, K = KB ? KB : D.nbasis;
+  const bool xdir = dir == 0, rk2 = D.dp == 2;
+  const int64_t ps = xdir ? S.pstride_u : S.pstride_v, bs = 6 * ps, step = xdir ? 1 : ld;
+  const double *W = (xdir ? D.wbu : D.wbv) + p * ps;
   const int row = D.unsteady ? min(D.ctl[1], D.max_steps - 1) : 0;   // steps completed
   const double *s1 = D.coef + (int64_t)row * 2 * K;   // coefficients at t_{n-1}
   const double *s0 = s1 + K;                          // at t_{n-2}
-  const double dto2 = 0.5 * D.dt;
-  const bool rk2 = D.dp == 2;
-  const int64_t bs_u = 6 * S.pstride_u, bs_v = 6 * S.pstride_v;
-  const double *Wu = D.wbu + p * S.pstride_u;
-  const double *Wv = D.wbv + p * S.pstride_v;
-  T *ua = reinterpret_cast<T *>(D.uavg) + p * S.pstride_u;
-  T *va = reinterpret_cast<T *>(D.vavg) + p * S.pstride_v;
-  T *us = D.usgn ? reinterpret_cast<T *>(D.usgn) + p * S.pstride_u : nullptr;
-  T *vs = D.vsgn ? reinterpret_cast<T *>(D.vsgn) + p * S.pstride_v : nullptr;
-  auto comb = [&](const double *W, int64_t bs, int64_t off, const double *s) {
-    if (K == 1) return wind_of_basis(s[0], W[off]);   // the same bits as the step's own (WIND)
-    double acc = 0.0;
-    for (int m = 0; m < K; ++m) acc += s[m] * W[m * bs + off];
-    return acc;
-  };
-  const int ne = N + 1;   // edges i0 .. iend
-  // one block per row of edges: x-edge rows c = 0 .. M-1 ([row][edge], edges i0 .. iend), then
-  // y-edge rows e = i0 .. iend ([edge][column], columns 0 .. M-1); threads run along the row,
-  // so consecutive threads take consecutive addresses and no index is divided
-  const int r = blockIdx.x;
-  if (r >= M + ne) return;                    // the grid covers the largest solve
-  const bool xdir = r < M;
-  const int len = xdir ? ne : M;
-  for (int t = threadIdx.x; t < len; t += blockDim.x) {
-    const int e = xdir ? t + i0 : r - M + i0;   // edge index along the flux direction
-    const int c = xdir ? r : t;                 // row (x-edges) / column (y-edges)
-    const int64_t bs = xdir ? bs_u : bs_v;
-    const double *W = xdir ? Wu : Wv;
-    const int64_t off = xdir ? (int64_t)c * ldu + e : (int64_t)e * ld + c;
-    const int64_t step = xdir ? 1 : ld;
-    const double rd = xdir ? 1.0 / D.dx : 1.0 / D.dy;
-    const double u = comb(W, bs, off, s1);
-    double avg = u;
-    if (rk2) {
-      auto ui = [&](int64_t o) {
-        const double un = comb(W, bs, o, s1);
-        const double uo = comb(W, bs, o, s0);
-        return 1.5 * un - 0.5 * uo;
-      };
-      const double a = (u * dto2) * rd;
-      if (u >= 0.0) avg = (1.0 - a) * ui(off) + a * ui(off - step);
-      else avg = -a * ui(off + step) + (1.0 + a) * ui(off);
-    }
-    if (xdir) { ua[off] = (T)avg; if (us) us[off] = (T)u; }
-    else { va[off] = (T)avg; if (vs) vs[off] = (T)u; }
+  // x-edges as [row 0 .. M-1][edge i0 .. iend], y-edges as [edge i0 .. iend][column 0 .. M-1]
+  const unsigned len = xdir ? N + 1 : M, total = (unsigned)M * (N + 1);
+  const unsigned first = (unsigned)blk * (BLOCK * kWindEdges) + threadIdx.x;
+  int64_t off[kWindEdges];
+  double u[kWindEdges], avg[kWindEdges];
+#pragma unroll
+  for (int k = 0; k < kWindEdges; ++k) {
+    const unsigned idx = min(first + k * BLOCK, total - 1);   // (past the last: its value again)
+    const unsigned r = idx / len, c = idx - r * len;
+    off[k] = xdir ? (int64_t)r * ldu + NG + c : (int64_t)(NG + r) * ld + c;
+    u[k] = avg[k] = wind_comb<KB>(W + off[k], bs, s1, K);
   }
+  if (rk2) {
+    double se[KB ? KB : kMaxBasis];                   // coefficients of the extrapolated wind
+#pragma unroll
+    for (int m = 0; m < (KB ? KB : kMaxBasis); ++m) se[m] = m < K ? 1.5 * s1[m] - 0.5 * s0[m] : 0.0;
+    const double dto2 = 0.5 * D.dt, rd = 1.0 / (xdir ? D.dx : D.dy);
+#pragma unroll
+    for (int k = 0; k < kWindEdges; ++k) {
+      const double a = (u[k] * dto2) * rd;
+      const double own = wind_comb<KB>(W + off[k], bs, se, K);
+      const double up = wind_comb<KB>(W + (u[k] >= 0.0 ? off[k] - step : off[k] + step), bs, se, K);
+      avg[k] = u[k] >= 0.0 ? (1.0 - a) * own + a * up : -a * up + (1.0 + a) * own;
+    }
+  }
+  T *ua = reinterpret_cast<T *>(xdir ? D.uavg : D.vavg) + p * ps;
+  T *us = reinterpret_cast<T *>(xdir ? D.usgn : D.vsgn);
+#pragma unroll
+  for (int k = 0; k < kWindEdges; ++k) {
+    if (first + k * BLOCK >= total) continue;
+    ua[off[k]] = (T)avg[k];
+    if (us) us[p * ps + off[k]] = (T)u[k];
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void wind_item(const Solve &S, int pd, int blk) {
+  const csadv_solve_desc &D = S.d;
+  if ((D.stop > 0 && D.ctl[1] >= D.stop) || D.ctl[0]) return;       // solve finished or halted
+  if (D.nbasis == 1) wind_edges<T, 1>(S, pd & 7, pd >> 3, blk);
+  else if (D.nbasis == 4) wind_edges<T, 4>(S, pd & 7, pd >> 3, blk);
+  else wind_edges<T, 0>(S, pd & 7, pd >> 3, blk);
+}
+
+// Workgroup b takes item b of the wind work list (wind_list: the time-dependent solves first, so
+// that a step launches only their items).
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void k_wind_avg(const Solve *solves, const int4 *list) {
+  const int4 it = list[blockIdx.x];
+  wind_item<T>(solves[it.x], it.y, it.z);
+}
+
+// A handle of one solve: the descriptor travels in the kernel arguments; grid (blocks, 12 = panel
+// and direction).
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void k_wind_avg1(const Solve one) {
+  const int y = blockIdx.y;
+  wind_item<T>(one, y % 6 + 8 * (y / 6), blockIdx.x);
 }
 
 // ------------------------------------------------------------------ diagnostics
@@ -789,18 +821,20 @@ int step_ghosts(csadv_t *h, hipStream_t st) {
   return CSADV_OK;
 }
 
+// The winds of the step: of the time-dependent solves, or of every solve (wind init).
 int wind_avg(csadv_t *h, hipStream_t st, bool all) {
-  const int ns = (int)h->desc.size();
-  bool any = all;
-  for (auto &d : h->desc) any = any || d.unsteady;
-  if (!any) return CSADV_OK;
-  int maxN = 0;
-  for (auto &d : h->desc) maxN = std::max(maxN, d.N);
-  const int blocks = (maxN + 2 * NG) + (maxN + 1);   // x-edge rows, then y-edge rows
-  if (h->dtype == CSADV_F64)
-    hipLaunchKernelGGL(k_wind_avg<double>, dim3(blocks, 6, ns), dim3(BLOCK), 0, st, h->dev, (int)all);
-  else
-    hipLaunchKernelGGL(k_wind_avg<float>, dim3(blocks, 6, ns), dim3(BLOCK), 0, st, h->dev, (int)all);
+  if (h->desc.size() == 1) {
+    const csadv_solve_desc &d = h->desc[0];
+    if (!all && !d.unsteady) return CSADV_OK;
+    const dim3 grid(wind_blocks(d.N), 12);
+    if (h->dtype == CSADV_F64) hipLaunchKernelGGL(k_wind_avg1<double>, grid, dim3(BLOCK), 0, st, h->host[0]);
+    else hipLaunchKernelGGL(k_wind_avg1<float>, grid, dim3(BLOCK), 0, st, h->host[0]);
+  } else {
+    const int n = all ? h->nwwork : h->nwunsteady;
+    if (!n) return CSADV_OK;
+    if (h->dtype == CSADV_F64) hipLaunchKernelGGL(k_wind_avg<double>, dim3(n), dim3(BLOCK), 0, st, h->dev, h->wwork);
+    else hipLaunchKernelGGL(k_wind_avg<float>, dim3(n), dim3(BLOCK), 0, st, h->dev, h->wwork);
+  }
   HIPCHK(h, hipGetLastError());
   return CSADV_OK;
 }
@@ -914,7 +948,16 @@ int csadv_update(csadv_t *h, const csadv_solve_desc *solves, int32_t nsolve, voi
   for (int s = 0; s < nsolve; ++s)
     h->wind1 = h->wind1 && solves[s].unsteady && solves[s].dp == 1 && solves[s].nbasis == 1;
   HIPCHK(h, hipMemcpyAsync(h->work, work.data(), sizeof(int4) * work.size(), hipMemcpyHostToDevice, st));
-  if (nsolve > 1) {                  // the ghost fill of a multi-solve handle reads its own list
+  if (nsolve > 1) {                  // the ghost fill and the winds of a multi-solve handle read their own lists
+    const std::vector<Item> ww = wind_list(h->host, h->nwunsteady);
+    if ((int)ww.size() != h->nwwork) {
+      if (h->wwork) (void)hipFree(h->wwork);
+      h->wwork = nullptr;
+      h->nwwork = 0;
+      HIPCHK(h, hipMalloc(&h->wwork, sizeof(int4) * ww.size()));
+      h->nwwork = (int)ww.size();
+    }
+    HIPCHK(h, hipMemcpyAsync(h->wwork, ww.data(), sizeof(int4) * ww.size(), hipMemcpyHostToDevice, st));
     const std::vector<Item> gw = ghost_list(h->host);
     if ((int)gw.size() != h->ngwork) {
       if (h->gwork) (void)hipFree(h->gwork);
@@ -1364,6 +1407,7 @@ void csadv_destroy(csadv_t *h) {
   if (h->dev) (void)hipFree(h->dev);
   if (h->work) (void)hipFree(h->work);
   if (h->gwork) (void)hipFree(h->gwork);
+  if (h->wwork) (void)hipFree(h->wwork);
   if (h->qsets) (void)hipFree(h->qsets);
   if (h->wsets) (void)hipFree(h->wsets);
   if (h->red) (void)hipFree(h->red);

@@ -19,10 +19,13 @@ struct csadv_s {
   Solve *dev = nullptr;           // device descriptors (caller-visible scratch is not used)
   int4 *work = nullptr;           // step work items
   int4 *gwork = nullptr;          // ghost-fill work items of a multi-solve handle (ghost_list)
+  int4 *wwork = nullptr;          // wind work items of a multi-solve handle (wind_list)
   FieldSet *qsets = nullptr;      // ghost-fill sets for the tracers
   FieldSet *wsets = nullptr;      // ghost-fill sets for the lat-lon centre winds
   int nwork = 0;
   int ngwork = 0;
+  int nwwork = 0;
+  int nwunsteady = 0;             // leading items of wwork: the time-dependent solves
   int tile = 0;
   int dtype = 0;
   int recon = 3;

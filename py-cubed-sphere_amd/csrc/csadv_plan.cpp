@@ -135,6 +135,21 @@ std::vector<Item> ghost_list(const std::vector<Solve> &solves) {
   return g;
 }
 
+std::vector<Item> wind_list(const std::vector<Solve> &solves, int &unsteady) {
+  std::vector<Item> w;
+  unsteady = 0;
+  for (int pass = 0; pass < 2; ++pass) {
+    for (int s = 0; s < (int)solves.size(); ++s) {
+      if ((solves[s].d.unsteady != 0) != (pass == 0)) continue;
+      const int blocks = wind_blocks(solves[s].d.N);
+      for (int pd = 0; pd < 12; ++pd)
+        for (int b = 0; b < blocks; ++b) w.push_back(Item{s, pd % 6 + 8 * (pd / 6), b, 0});
+    }
+    if (pass == 0) unsteady = (int)w.size();
+  }
+  return w;
+}
+
 int partials_per_tracer(int N, int tile) {
   if (tile < 0 || tile >= kNumTiles || N < 1) return CSADV_E_ARG;
   int sw, ns, sl, nsg;

@@ -25,6 +25,7 @@ constexpr int kXcds = 8;             // MI355X: 8 XCDs; workgroup b is dispatche
 constexpr int STRIP_MAX = WAVE - 6;  // interior columns of one wavefront (3-cell halo each side)
 constexpr int kDiagBlocks = 256;     // blocks of a diagnostics reduction (partials per tracer)
 constexpr int kDiagWords = 8;        // doubles per diagnostics partial
+constexpr int kWindEdges = 4;        // edges of one thread of the wind kernel
 constexpr int kMaxTracers = 64;      // tracers per solve
 
 // tile id -> rows per wavefront segment (the strip width is always the widest that fits)
@@ -139,6 +140,16 @@ std::vector<Item> work_list(const std::vector<Solve> &solves, int group = 1);
 // blocks of tracer 0 first) as in a dense (blocks, solves, tracers) grid, without that grid's
 // blocks past a solve's cells or tracers.
 std::vector<Item> ghost_list(const std::vector<Solve> &solves);
+
+// Blocks of one panel's winds of one direction: its (N + 8)(N + 1) edges, kWindEdges per thread.
+inline int wind_blocks(int N) {
+  const int64_t per = (int64_t)BLOCK * kWindEdges, edges = (int64_t)(N + 2 * NG) * (N + 1);
+  return (int)((edges + per - 1) / per);
+}
+
+// The winds' work list of a multi-solve handle: (solve, panel + 8 * direction, block) of every
+// solve, the time-dependent solves first (the first `unsteady` items).
+std::vector<Item> wind_list(const std::vector<Solve> &solves, int &unsteady);
 
 // Sizes of the public entry points (see include/csadv.h).
 int partials_per_tracer(int N, int tile);
