@@ -145,6 +145,98 @@ __device__ __forceinline__ T upwind(bool up, T LrA, T LrB, T Lq6, const Parab<T>
   return f;
 }
 
+// Upwind flux in weighted form.  With c the Courant number of an edge, s = c when the wind there
+// is non-negative and -c otherwise, A the upwind cell's edge value at this edge, D its other edge
+// value and q its mean (A, D, q with the MT-0 metric on them), CW84's flux (src/flux.py:28-70) is
+//   F dt/dx = c (al A + be D + ga q),  al = (1 - s)^2,  be = -s (1 - s),  ga = s (3 - 2 s),
+// so every edge is three products with weights that depend on the wind and the metric only: they
+// are formed once per edge and serve both passes of the split and every tracer.
+// PPM-0 and PPM-PL07 are linear in the window, so their edge values split into a part symmetric
+// and a part antisymmetric about the cell, A, D = e +- o, with
+//   e = k3 q + k1 (S1 + r S2),  o = h1 (D1 + t D2),  S, D the sums and differences of the
+// neighbours at distance 1 and 2: a cell is then six operations (where its two edge values and
+// their parabola took eighteen) and k1, k3, h1 go into the weights.
+template <int RECON> struct Lin {
+  static constexpr bool on = RECON == 1 || RECON == 3;
+  static constexpr double k3 = RECON == 1 ? 7.0 / 12.0 : 47.0 / 60.0, k1 = RECON == 1 ? 0.25 : 14.0 / 120.0;
+  static constexpr double r = RECON == 1 ? -1.0 / 6.0 : -1.0 / 14.0, h1 = 1.0 / 3.0, t = -1.0 / 8.0;
+};
+
+// What an edge takes from a cell: linear schemes a = S1 + r S2, b = D1 + t D2, the others the edge
+// values a = q_L, b = q_R; q the mean.
+template <typename T>
+struct Cell {
+  T a, b, q;
+};
+
+template <typename T, int RECON>
+__device__ __forceinline__ Cell<T> cell_of(T m2, T m1, T c0, T p1, T p2) {
+  using L = Lin<RECON>;
+  Cell<T> c;
+  c.q = c0;
+  if constexpr (L::on) {
+    c.a = __builtin_elementwise_fma(T(L::r), p2 + m2, p1 + m1);
+    c.b = __builtin_elementwise_fma(T(L::t), p2 - m2, p1 - m1);
+  } else {
+    recon_edges<T, RECON>(m2, m1, c0, p1, p2, c.a, c.b);
+  }
+  return c;
+}
+
+// An edge's weights: of the upwind cell's mean (w0) and, linear schemes, its a and b (w1, w2), the
+// others its A and D; up: the upwind cell is the left one.
+template <typename T>
+struct EdgeW {
+  T w0, w1, w2;
+  bool up;
+};
+
+// The weights of an edge with Courant number c (s as above), gA / gD the edge metrics at the edge
+// and at the upwind cell's other edge, gq its centre metric (MT-0); MT-PL07 (mt0 false) takes the
+// edge's metric gA on the whole flux.  Multiply-adds are written as fma where they fuse, so that
+// the bits do not depend on the surrounding code.
+template <typename T, int RECON>
+__device__ __forceinline__ EdgeW<T> edge_weights(bool up, T c, T s, T gA, T gD, T gq, bool mt0) {
+  using L = Lin<RECON>;
+  const T om = T(1) - s, ga = s * __builtin_elementwise_fma(T(-2), s, T(3));
+  EdgeW<T> w;
+  w.up = up;
+  if (mt0) {
+    const T ag = (om * om) * gA, t = s * om;
+    if constexpr (L::on) {
+      const T P = __builtin_elementwise_fma(-t, gD, ag), M = __builtin_elementwise_fma(t, gD, ag);
+      w.w0 = c * __builtin_elementwise_fma(T(L::k3), P, ga * gq);
+      w.w1 = (c * T(L::k1)) * P;
+      w.w2 = (s * T(L::h1)) * M;
+    } else {
+      w.w0 = c * (ga * gq);
+      w.w1 = c * ag;
+      w.w2 = -c * (t * gD);
+    }
+  } else {
+    const T cg = c * gA;
+    if constexpr (L::on) {
+      const T P = om * (om - s);
+      w.w0 = cg * __builtin_elementwise_fma(T(L::k3), P, ga);
+      w.w1 = (cg * T(L::k1)) * P;
+      w.w2 = ((s * gA) * T(L::h1)) * om;
+    } else {
+      w.w0 = cg * ga;
+      w.w1 = cg * (om * om);
+      w.w2 = -cg * (s * om);
+    }
+  }
+  return w;
+}
+
+// Flux (times dt/dx) of an edge from the cells on its left and right.
+template <typename T, int RECON>
+__device__ __forceinline__ T edge_flux(const EdgeW<T> &w, T la, T lb, T lq, const Cell<T> &R) {
+  constexpr bool lin = Lin<RECON>::on;
+  const T q = w.up ? lq : R.q, x = w.up ? (lin ? la : lb) : R.a, y = w.up ? (lin ? lb : la) : R.b;
+  return __builtin_elementwise_fma(w.w2, y, __builtin_elementwise_fma(w.w1, x, w.w0 * q));
+}
+
 // Whole-wavefront DPP lane shifts (one v_mov_b32_dpp per dword, no LDS round trip):
 // from_left(v) is v of lane-1, from_right(v) is v of lane+1; the end lane without a source
 // (lane 0, resp. lane 63) reads zero.  The step kernel only ever stores results of lanes
@@ -211,6 +303,13 @@ __device__ __forceinline__ T upwind_x(bool up, const Parab<T> &c, T cc, T gl, T 
   return up ? from_l : fl;
 }
 
+// Flux through the left edge of each lane's cell along the wavefront (x): the left cell's a and b
+// by lane shifts, its mean from the window (m1).
+template <typename T, int RECON>
+__device__ __forceinline__ T edge_flux_x(const EdgeW<T> &w, const Cell<T> &c, T m1) {
+  return edge_flux<T, RECON>(w, from_left(c.a), from_left(c.b), m1, c);
+}
+
 // Element idx of an array whose base is wave-uniform: the byte offset stays 32-bit so that
 // the load takes the scalar-base + vector-offset form (callers keep idx * sizeof(T) < 4 GiB).
 // Every array handed to the library is device global memory, so the access is made in the
@@ -260,6 +359,24 @@ __device__ __forceinline__ T split_update(int split, T Q, T dF, T g, T rg, T c1,
   if (split == 2) return (Q * g + T(0.5) * dF + T(0.5) * (c1 - c2) * Q) * rg;
   return T(0.5) * (Q + (Q + dF) / (T(1.0) - (c1 - c2)));
 }
+
+// The split's half-step of one cell (src/discrete_operators.py:49-73) in two parts: a factor that
+// depends on the winds and the metric only (shared by the tracers), and the update with it.
+// dc = c1 - c2, the difference of the metric-weighted Courant numbers of the cell's edges.
+//   AVLT: Q + dF / (2 g);  L04: Q + (dF + dc Q) / (2 g);  PL07: Q / 2 + (Q + dF) / (2 (1 - dc))
+template <typename T, int SPLIT>
+__device__ __forceinline__ T half_factor(T rg, T dc) {
+  if constexpr (SPLIT == 3) return T(0.5) / (T(1) - dc);
+  else return T(0.5) * rg;
+}
+template <typename T, int SPLIT>
+__device__ __forceinline__ T half_step(T Q, T dF, T h, T dc) {
+  if constexpr (SPLIT == 1) return __builtin_elementwise_fma(h, dF, Q);
+  else if constexpr (SPLIT == 2) return __builtin_elementwise_fma(h, __builtin_elementwise_fma(dc, Q, dF), Q);
+  else return __builtin_elementwise_fma(h, Q + dF, T(0.5) * Q);
+}
+__device__ __forceinline__ float fabs_t(float v) { return fabsf(v); }
+__device__ __forceinline__ double fabs_t(double v) { return fabs(v); }
 
 // MF-AF (src/edges_treatment.py:231-278) on boundary cells of a new state: F holds the second
 // pass's fluxes through the 24 panel sides ([panel][E, W, N, S][N], scaled by dt/dx as the step

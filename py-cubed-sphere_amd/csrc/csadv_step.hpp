@@ -92,12 +92,12 @@ struct March {
   //                   guw x-edge metric, gvr gv at y-edge r-2
   //   computed, row r: qw Q (corrected), xw the split half-step Qx, sw (FP32) Q as stored
   //   (per tracer: qr, qar, qw, xw, sw, the flux carries and the partial sum)
-  T qr[NT][RS], gfr[RS], qar[NT][RS], vr[RS], vsr[RS];
-  T qw[NT][RD], xw[NT][RD], gcw[RD], rgw[RD], uw[RD], usw[RD], guw[RD], gvr[RD];
-  T sw[NT][RD];
-  T g1prev[NT], g2prev[NT], vprev;
-  // row y-4 as the left (upwind) cell of edge y-3: Q, Qx
-  T pa_A[NT], pa_B[NT], pa_q6[NT], pb_A[NT], pb_B[NT], pb_q6[NT];
+  T qr[NT][RS], gfr[RS], qar[NT][RS], ur[RS], usr[RS], gur[RS], vr[RS], vsr[RS];
+  T qw[NT][RD], xw[NT][RD], sw[NT][RD], gcw[RD], rgw[RD], gvr[RD];
+  T x0[RD], x1[RD], x2[RD];
+  bool xup[RD];
+  T g1prev[NT], g2prev[NT], hyprev;
+  Cell<T> pa[NT], pb[NT];          // row y-4 as the left cell of edge y-3: Q, Qx
   double part[NT];
 
   // Inputs of row y into ring slot SLOT.  SPEC: also read Q from the other state buffer (Qa),
@@ -106,13 +106,13 @@ struct March {
   __device__ __forceinline__ void load(int y) {
     const int yc = min(y, M - 1);
     const uint32_t o = (uint32_t)(yc * ld + xc), ou = (uint32_t)(yc * ldu + xe);
-    if constexpr (WIND) uw[SLOT] = T(wind_of_basis(ws, ld_at(WU, ou)));
-    else uw[SLOT] = ld_at(U, ou);
-    if constexpr (RK2) usw[SLOT] = ld_at(US, ou);
-    guw[SLOT] = ld_at(gu, ou);
+    constexpr int SS = SLOT % RS;          // state slot
+    if constexpr (WIND) ur[SS] = T(wind_of_basis(ws, ld_at(WU, ou)));
+    else ur[SS] = ld_at(U, ou);
+    if constexpr (RK2) usr[SS] = ld_at(US, ou);
+    gur[SS] = ld_at(gu, ou);
     gcw[SLOT] = ld_at(gc, o);
     rgw[SLOT] = ld_at(rgc, o);
-    constexpr int SS = SLOT % RS;          // state slot
     gfr[SS] = ld_at(gfix, o);
     // Q of every lane, at the clamped row and column (rows past ylast are requested too): no
     // branch around the load, and the value outside the stencils' reach is replaced by zero
@@ -143,10 +143,6 @@ struct March {
   // the panel's 3-cell halo and interior; the array's outer ghost layer is never read)
   __device__ __forceinline__ bool reach(int y) const { return need_col && y >= 1 && y < iend + 3; }
 
-  // the upwind-side winds of the row in a slot (RK1: the winds themselves)
-  __device__ __forceinline__ T wind_sign(int slot) const { return RK2 ? usw[slot] : uw[slot]; }
-  __device__ __forceinline__ T vwind_sign(int slot) const { return RK2 ? vsr[slot] : vr[slot]; }
-
   // every cell the stencils read carries the mass-fixer correction total C: Q = S + C gfix,
   // gfix being g inside the panel and, at a ghost cell, the weighted metric of the cells its
   // value was interpolated from (in the solve's precision: C gfix is ~1e-6 of q at most, so
@@ -154,8 +150,8 @@ struct March {
   // outside the stencils' reach hold 0 + C gfix, which no stored cell reads.
   // (with no correction total, cf = 0 and q + 0 gfix = q: no branch on the mass fixer)
   __device__ __forceinline__ T corrected(T raw, T gf, int t) const {
-    if constexpr (std::is_same<T, float>::value) return (raw + off[t]) + T(cf[t]) * gf;
-    else return raw + T(cf[t]) * gf;
+    if constexpr (std::is_same<T, float>::value) return __builtin_elementwise_fma(T(cf[t]), gf, raw + off[t]);
+    else return __builtin_elementwise_fma(T(cf[t]), gf, raw);
   }
 
   // Iteration y in phase K.  STAGE: how much of the column stage has begun, fixed by the row's
@@ -176,54 +172,48 @@ struct March {
     }
     const T gvm1 = gvr[s4], gv0 = gvr[s5], gvp1 = gvr[s0];   // gv at y-edges y-4, y-3, y-2
     T out = T(0);
-    // ---- column stage: parabolas of row y-3, y-edge e = y-3, output row r = y-4
+    // ---- column stage: cells of row y-3, y-edge e = y-3, output row r = y-4
     if constexpr (STAGE >= 1) {
-      const T gce = gcw[s3];
-      Parab<T> a[NT], b[NT];
+      Cell<T> a[NT], b[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        a[t] = parabola<T, RECON>(qw[t][s1], qw[t][s2], qw[t][s3], qw[t][s4], qw[t][s5], gv0, gvp1, gce, mt0);
-        b[t] = parabola<T, RECON>(xw[t][s1], xw[t][s2], xw[t][s3], xw[t][s4], xw[t][s5], gv0, gvp1, gce, mt0);
+        a[t] = cell_of<T, RECON>(qw[t][s1], qw[t][s2], qw[t][s3], qw[t][s4], qw[t][s5]);
+        b[t] = cell_of<T, RECON>(xw[t][s1], xw[t][s2], xw[t][s3], xw[t][s4], xw[t][s5]);
       }
       if constexpr (STAGE >= 2) {
-        const T v = vr[ss];
-        const bool vup = vwind_sign(ss) >= T(0);
-        const T cy = v * dtdy;
+        const T cy = vr[ss] * dtdy;
+        const bool vup = (RK2 ? vsr[ss] : vr[ss]) >= T(0);
+        const EdgeW<T> wy = edge_weights<T, RECON>(vup, cy, RK2 ? (vup ? cy : -cy) : fabs_t(cy), gv0, vup ? gvm1 : gvp1,
+                                                   vup ? gcw[s2] : gcw[s3], mt0);
+        T hy = T(0);
+        if constexpr (split != 1) hy = gv0 * cy;
         T g1[NT], g2[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          g1[t] = upwind<T>(vup, pa_A[t], pa_B[t], pa_q6[t], a[t], cy, gv0, mt0);     // times dt/dy
-          g2[t] = upwind<T>(vup, pb_A[t], pb_B[t], pb_q6[t], b[t], cy, gv0, mt0);
+          g1[t] = edge_flux<T, RECON>(wy, pa[t].a, pa[t].b, pa[t].q, a[t]);     // times dt/dy
+          g2[t] = edge_flux<T, RECON>(wy, pb[t].a, pb[t].b, pb[t].q, b[t]);
         }
         if constexpr (STAGE >= 3) {
-          const T gcm = gcw[s2];               // row y-4
-          T d1 = T(0), d2 = T(0);
-          if (split != 1) {
-            d1 = gv0 * cy;
-            d2 = gvm1 * (vprev * dtdy);
-          }
-          const T rg = rgw[s2];
-          const T ur = uw[s2];
-          const bool urp = wind_sign(s2) >= T(0);
-          const T gur = guw[s2];
+          const T rg = rgw[s2];                // row y-4
+          const T h = half_factor<T, SPLIT>(rg, hy - hyprev);
+          const EdgeW<T> wx{x0[s2], x1[s2], x2[s2], xup[s2]};
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
             const T dG1 = g1prev[t] - g1[t];
-            const T qy = split_update<T>(split, qw[t][s2], dG1, gcm, rg, d1, d2);
+            const T qy = half_step<T, SPLIT>(qw[t][s2], dG1, h, hy - hyprev);
             T qy_m2, qy_m1, qy_p1, qy_p2;
             xwindow<T, XPULL>(qy, am2, am1, ap1, ap2, qy_m2, qy_m1, qy_p1, qy_p2);
-            const Parab<T> c = parabola<T, RECON>(qy_m2, qy_m1, qy, qy_p1, qy_p2, gur, from_right(gur), gcm, mt0);
-            const T f2 = upwind_x<T>(urp, c, ur * dtdx, gur, from_right(gur), mt0);
+            const T f2 = edge_flux_x<T, RECON>(wx, cell_of<T, RECON>(qy_m2, qy_m1, qy, qy_p1, qy_p2), qy_m1);
             const T dF2 = f2 - from_right(f2);
             const T dG2 = g2prev[t] - g2[t];
             // div = -(dF2 + dG2) / (dt g);  Q - dt div = Q + (dF2 + dG2) / g
             const T flx = dF2 + dG2;
             // the correction total stays out of the stored state: S(n+1) = S(n) + flux
             if constexpr (EXACT) {
-              out = (qw[t][s2] + flx * rg) - T(cf[t]) * gcm;
+              out = __builtin_elementwise_fma(flx, rg, sw[t][s2]);
               if (out_lane) part[t] -= (double)flx;   // used with MF-PR only
             } else if (out_lane) {
-              st_at(Qo[t], (uint32_t)((y - 4) * ld + x), sw[t][s2] + flx * rg);
+              st_at(Qo[t], (uint32_t)((y - 4) * ld + x), __builtin_elementwise_fma(flx, rg, sw[t][s2]));
               part[t] -= (double)flx;
             }
             if (fside[0]) {   // MF-AF: cube-edge fluxes of output row r = y - 4 (f2: left edge of the lane's cell)
@@ -240,42 +230,44 @@ struct March {
           g1prev[t] = g1[t];
           g2prev[t] = g2[t];
         }
-        vprev = v;
+        hyprev = hy;
       }
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        pa_A[t] = a[t].rA; pa_B[t] = a[t].rB; pa_q6[t] = a[t].q6;
-        pb_A[t] = b[t].rA; pb_B[t] = b[t].rB; pb_q6[t] = b[t].q6;
+        pa[t] = a[t];
+        pb[t] = b[t];
       }
     }
     // ---- row stage: row y.  Qx of the march's last row, ylast, is read by no stencil (the
     // last parabola row is ylast-3, whose window ends at ylast-1).  FP32, bound by issue, skips
-    // it by a wave-uniform branch (2-3% of the launch).  FP64 does not: the branch changes the
-    // code layout, and the one-solve and multi-solve kernels then round alike only when
-    // multiply-adds are fused per expression, which costs the latency-bound FP64 kernel 1.5-2%
+    // it by a wave-uniform branch (2-3% of the launch).
     if (!std::is_same<T, float>::value || STAGE < 3 || y < ylast) {
-      const T u = uw[s0], gu0 = guw[s0], gc0 = gcw[s0];
-      const bool up = wind_sign(s0) >= T(0);
-      const T gup1 = from_right(gu0);
-      T c1 = T(0), c2 = T(0);
-      if (split != 1) {
-        c1 = gup1 * (from_right(u) * dtdx);
-        c2 = gu0 * (u * dtdx);
+      const T u = ur[ss], gu0 = gur[ss], gc0 = gcw[s0], cx = u * dtdx;
+      const bool up = (RK2 ? usr[ss] : u) >= T(0);
+      // (the lane shifts before the selects: every lane takes part in them)
+      const T gul = from_left(gu0), gur1 = from_right(gu0), gcl = from_left(gc0);
+      const EdgeW<T> wx = edge_weights<T, RECON>(up, cx, RK2 ? (up ? cx : -cx) : fabs_t(cx), gu0, up ? gul : gur1,
+                                                 up ? gcl : gc0, mt0);
+      x0[s0] = wx.w0; x1[s0] = wx.w1; x2[s0] = wx.w2; xup[s0] = up;
+      T dh = T(0);
+      if constexpr (split != 1) {
+        const T hx0 = gu0 * cx;
+        dh = from_right(hx0) - hx0;
       }
+      const T h = half_factor<T, SPLIT>(rgw[s0], dh);
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         T q_m2, q_m1, q_p1, q_p2;
         xwindow<T, XPULL>(q[t], am2, am1, ap1, ap2, q_m2, q_m1, q_p1, q_p2);
-        const Parab<T> c = parabola<T, RECON>(q_m2, q_m1, q[t], q_p1, q_p2, gu0, gup1, gc0, mt0);
-        const T f1 = upwind_x<T>(up, c, u * dtdx, gu0, gup1, mt0);
+        const T f1 = edge_flux_x<T, RECON>(wx, cell_of<T, RECON>(q_m2, q_m1, q[t], q_p1, q_p2), q_m1);
         const T dF1 = f1 - from_right(f1);
-        xw[t][s0] = split_update<T>(split, q[t], dF1, gc0, rgw[s0], c1, c2);
+        xw[t][s0] = half_step<T, SPLIT>(q[t], dF1, h, dh);
       }
     }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       qw[t][s0] = q[t];
-      if constexpr (std::is_same<T, float>::value) sw[t][s0] = raw[t];
+      sw[t][s0] = raw[t];
     }
     // rows past ylast are read in bounds (clamped rows, masked Q) and never used
     load<false, sl(K, PF)>(y + PF);
@@ -294,10 +286,13 @@ struct March {
   // buffers (Q = q0, Qa = q1), the rest from the step-invariant tables and winds.
   __device__ __forceinline__ void start() {
 #pragma unroll
-    for (int k = 0; k < RD; ++k) gcw[k] = rgw[k] = uw[k] = usw[k] = guw[k] = gvr[k] = T(0);
+    for (int k = 0; k < RD; ++k) {
+      gcw[k] = rgw[k] = gvr[k] = x0[k] = x1[k] = x2[k] = T(0);
+      xup[k] = false;
+    }
 #pragma unroll
-    for (int k = 0; k < RS; ++k) gfr[k] = vr[k] = vsr[k] = T(0);
-    vprev = T(0);   // gv is complete from y = tj-1 on; the column stage starts at tj+2
+    for (int k = 0; k < RS; ++k) gfr[k] = ur[k] = usr[k] = gur[k] = vr[k] = vsr[k] = T(0);
+    hyprev = T(0);   // gv is complete from y = tj-1 on; the column stage starts at tj+2
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
 #pragma unroll
@@ -305,7 +300,7 @@ struct March {
 #pragma unroll
       for (int k = 0; k < RS; ++k) qr[t][k] = qar[t][k] = T(0);
       g1prev[t] = g2prev[t] = T(0);
-      pa_A[t] = pa_B[t] = pa_q6[t] = pb_A[t] = pb_B[t] = pb_q6[t] = T(0);
+      pa[t] = pb[t] = Cell<T>{T(0), T(0), T(0)};
       part[t] = 0.0;
     }
     // y0 = tj - 3 has phase 0; ylast - y0 = ny + 6 >= PF: every initial row exists
