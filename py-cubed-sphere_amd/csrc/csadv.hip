@@ -531,6 +531,24 @@ __device__ __forceinline__ double wind_comb(const double *W, int64_t bs, const d
   }
 }
 
+// The flux-table entry of an edge (x: edge e of row r; y: edge r of column e) with upwind-side
+// wind u and averaged wind avg, formed in FP64 and rounded once.
+template <typename T>
+__device__ __forceinline__ FluxEntry<T> flux_entry(const csadv_solve_desc &D, bool xdir, int64_t r, int64_t e, double u,
+                                                   double avg) {
+#pragma clang fp contract(off)
+  const bool up = u >= 0.0, mt0 = D.split != 3;
+  const T *gm = reinterpret_cast<const T *>(xdir ? D.gu : D.gv);
+  const int64_t row = xdir ? D.ldu : D.ld, step = xdir ? 1 : D.ld, o = r * row + e, oc = r * D.ld + e;
+  const double gA = gm[o], gD = gm[up ? o - step : o + step], gq = D.gc64[up ? oc - step : oc];
+  const double c = avg * (D.dt / (xdir ? D.dx : D.dy)), s = up ? c : -c;
+  EdgeW<double> w;
+  if (D.recon == 3) w = edge_weights<double, 3>(up, c, s, gA, gD, gq, mt0);
+  else if (D.recon == 1) w = edge_weights<double, 1>(up, c, s, gA, gD, gq, mt0);
+  else w = edge_weights<double, 2>(up, c, s, gA, gD, gq, mt0);
+  return {(T)w.w0, (T)w.w1, tag_low((T)w.w2, up), (T)(gA * c)};
+}
+
 // Block blk of the x-edges (dir 0) or y-edges (dir 1) of panel p.
 template <typename T, int KB>
 __device__ __forceinline__ void wind_edges(const Solve &S, int p, int dir, int blk) {
@@ -574,6 +592,14 @@ __device__ __forceinline__ void wind_edges(const Solve &S, int p, int dir, int b
     if (first + k * BLOCK >= total) continue;
     ua[off[k]] = (T)avg[k];
     if (us) us[p * ps + off[k]] = (T)u[k];
+    if (S.ftx) {
+      const int nw = flux_words(D.split), row = xdir ? ldu : ld;
+      const int64_t r = off[k] / row, e = off[k] - r * row;
+      const FluxEntry<T> f = flux_entry<T>(D, xdir, r, e, u[k], avg[k]);
+      T *o = reinterpret_cast<T *>(xdir ? S.ftx : S.fty) + (p * ps + off[k]) * nw;
+      o[0] = f.w0; o[1] = f.w1; o[2] = f.w2;
+      if (nw == 4) o[3] = f.h;
+    }
   }
 }
 
@@ -825,7 +851,7 @@ int step_ghosts(csadv_t *h, hipStream_t st) {
 int wind_avg(csadv_t *h, hipStream_t st, bool all) {
   if (h->desc.size() == 1) {
     const csadv_solve_desc &d = h->desc[0];
-    if (!all && !d.unsteady) return CSADV_OK;
+    if (!all && (!d.unsteady || own_wind(d))) return CSADV_OK;
     const dim3 grid(wind_blocks(d.N), 12);
     if (h->dtype == CSADV_F64) hipLaunchKernelGGL(k_wind_avg1<double>, grid, dim3(BLOCK), 0, st, h->host[0]);
     else hipLaunchKernelGGL(k_wind_avg1<float>, grid, dim3(BLOCK), 0, st, h->host[0]);
@@ -836,6 +862,59 @@ int wind_avg(csadv_t *h, hipStream_t st, bool all) {
     else hipLaunchKernelGGL(k_wind_avg<float>, dim3(n), dim3(BLOCK), 0, st, h->dev, h->wwork);
   }
   HIPCHK(h, hipGetLastError());
+  return CSADV_OK;
+}
+
+// The launch plan of the handle's descriptors and flux tables: each solve's mode, the work lists,
+// and the device copy of all of it.
+int upload_plan(csadv_t *h, hipStream_t st) {
+  const int nsolve = (int)h->host.size();
+  for (int s = 0; s < nsolve; ++s) {
+    Solve &S = h->host[s];
+    const csadv_solve_desc &d = h->desc[s];
+    S.mode = own_wind(d) ? kWind : h->ftab[s] ? kTab : d.dp == 2 ? kRk2 : kRk1;
+    S.ftx = S.fty = nullptr;
+    if (S.mode == kTab) {
+      S.ftx = h->ftab[s];
+      S.fty = static_cast<char *>(h->ftab[s]) + flux_x_elems(d.N, d.split) * (d.dtype == CSADV_F64 ? 8 : 4);
+    }
+    h->mode = s == 0 || h->mode == S.mode ? S.mode : (h->rk2 ? kMixed2 : kMixed);
+  }
+  // workgroup b runs on XCD b % kXcds (the list interleaves one band of row segments per XCD)
+  static_assert(sizeof(Item) == sizeof(int4), "work items are read as int4");
+  // (the FP32 multi-solve step kernel marches two tracers per item: kStepGroup in csadv_step.hpp)
+  const int group = (!h->general && h->dtype == CSADV_F32 && nsolve > 1) ? 2 : 1;
+  const std::vector<Item> work = work_list(h->host, group);
+  if ((int)work.size() != h->nwork) {
+    if (h->work) (void)hipFree(h->work);
+    h->work = nullptr;
+    HIPCHK(h, hipMalloc(&h->work, sizeof(int4) * work.size()));
+    h->nwork = (int)work.size();
+  }
+  h->mfaf = false;
+  for (int s = 0; s < nsolve; ++s) h->mfaf = h->mfaf || (!h->general && h->desc[s].mf == 2);
+  HIPCHK(h, hipMemcpyAsync(h->work, work.data(), sizeof(int4) * work.size(), hipMemcpyHostToDevice, st));
+  if (nsolve > 1) {                  // the ghost fill and the winds of a multi-solve handle read their own lists
+    const std::vector<Item> ww = wind_list(h->host, h->nwunsteady);
+    if ((int)ww.size() != h->nwwork) {
+      if (h->wwork) (void)hipFree(h->wwork);
+      h->wwork = nullptr;
+      h->nwwork = 0;
+      HIPCHK(h, hipMalloc(&h->wwork, sizeof(int4) * ww.size()));
+      h->nwwork = (int)ww.size();
+    }
+    HIPCHK(h, hipMemcpyAsync(h->wwork, ww.data(), sizeof(int4) * ww.size(), hipMemcpyHostToDevice, st));
+    const std::vector<Item> gw = ghost_list(h->host);
+    if ((int)gw.size() != h->ngwork) {
+      if (h->gwork) (void)hipFree(h->gwork);
+      h->gwork = nullptr;
+      HIPCHK(h, hipMalloc(&h->gwork, sizeof(int4) * gw.size()));
+      h->ngwork = (int)gw.size();
+    }
+    HIPCHK(h, hipMemcpyAsync(h->gwork, gw.data(), sizeof(int4) * gw.size(), hipMemcpyHostToDevice, st));
+  }
+  HIPCHK(h, hipMemcpyAsync(h->dev, h->host.data(), sizeof(Solve) * nsolve, hipMemcpyHostToDevice, st));
+  HIPCHK(h, hipStreamSynchronize(st));   // the lists above are host memory of this call
   return CSADV_OK;
 }
 
@@ -850,6 +929,10 @@ int csadv_partials_per_tracer(int32_t N, int32_t tile) { return partials_per_tra
 int csadv_work_bytes(int32_t N, int32_t dtype, int64_t *bytes) { return work_bytes(N, dtype, bytes); }
 
 int csadv_tile_rows(int32_t tile) { return tile_rows(tile); }
+
+int csadv_flux_table_bytes(int32_t N, int32_t dtype, int32_t split, int64_t *bytes) {
+  return flux_table_bytes(N, dtype, split, bytes);
+}
 
 int csadv_create(const csadv_solve_desc *solves, int32_t nsolve, int32_t tile, csadv_t **out) {
   if (!out) return CSADV_E_ARG;
@@ -881,6 +964,7 @@ int csadv_create(const csadv_solve_desc *solves, int32_t nsolve, int32_t tile, c
   *out = h;
   if (rc != CSADV_OK) return fail(h, rc, msg);
   h->done.assign(nsolve, 0);
+  h->ftab.assign(nsolve, nullptr);
   h->red_tracers = maxtr;
   hipError_t e;
   if ((e = hipMalloc(&h->dev, sizeof(Solve) * nsolve)) != hipSuccess ||
@@ -931,43 +1015,8 @@ int csadv_update(csadv_t *h, const csadv_solve_desc *solves, int32_t nsolve, voi
     const int rc = check_compatible(solves, nsolve, msg);
     if (rc != CSADV_OK) return fail(h, rc, msg);
   }
-  // workgroup b runs on XCD b % kXcds (the list interleaves one band of row segments per XCD)
-  static_assert(sizeof(Item) == sizeof(int4), "work items are read as int4");
-  // (the FP32 multi-solve step kernel marches two tracers per item: kStepGroup in csadv_step.hpp)
-  const int group = (!h->general && h->dtype == CSADV_F32 && nsolve > 1) ? 2 : 1;
-  const std::vector<Item> work = work_list(h->host, group);
-  if ((int)work.size() != h->nwork) {
-    if (h->work) (void)hipFree(h->work);
-    h->work = nullptr;
-    HIPCHK(h, hipMalloc(&h->work, sizeof(int4) * work.size()));
-    h->nwork = (int)work.size();
-  }
-  h->mfaf = false;
-  for (int s = 0; s < nsolve; ++s) h->mfaf = h->mfaf || (!h->general && solves[s].mf == 2);
-  h->wind1 = !h->general;
-  for (int s = 0; s < nsolve; ++s)
-    h->wind1 = h->wind1 && solves[s].unsteady && solves[s].dp == 1 && solves[s].nbasis == 1;
-  HIPCHK(h, hipMemcpyAsync(h->work, work.data(), sizeof(int4) * work.size(), hipMemcpyHostToDevice, st));
-  if (nsolve > 1) {                  // the ghost fill and the winds of a multi-solve handle read their own lists
-    const std::vector<Item> ww = wind_list(h->host, h->nwunsteady);
-    if ((int)ww.size() != h->nwwork) {
-      if (h->wwork) (void)hipFree(h->wwork);
-      h->wwork = nullptr;
-      h->nwwork = 0;
-      HIPCHK(h, hipMalloc(&h->wwork, sizeof(int4) * ww.size()));
-      h->nwwork = (int)ww.size();
-    }
-    HIPCHK(h, hipMemcpyAsync(h->wwork, ww.data(), sizeof(int4) * ww.size(), hipMemcpyHostToDevice, st));
-    const std::vector<Item> gw = ghost_list(h->host);
-    if ((int)gw.size() != h->ngwork) {
-      if (h->gwork) (void)hipFree(h->gwork);
-      h->gwork = nullptr;
-      HIPCHK(h, hipMalloc(&h->gwork, sizeof(int4) * gw.size()));
-      h->ngwork = (int)gw.size();
-    }
-    HIPCHK(h, hipMemcpyAsync(h->gwork, gw.data(), sizeof(int4) * gw.size(), hipMemcpyHostToDevice, st));
-  }
-  HIPCHK(h, hipMemcpyAsync(h->dev, h->host.data(), sizeof(Solve) * nsolve, hipMemcpyHostToDevice, st));
+  const int rc = upload_plan(h, st);
+  if (rc) return rc;
   HIPCHK(h, hipMemcpyAsync(h->qsets, sets.data(), sizeof(FieldSet) * nsolve, hipMemcpyHostToDevice, st));
   // steps already completed by each solve (a handle may be built over solves that have run)
   std::vector<int32_t> ctl(4 * nsolve);
@@ -976,6 +1025,31 @@ int csadv_update(csadv_t *h, const csadv_solve_desc *solves, int32_t nsolve, voi
   HIPCHK(h, hipStreamSynchronize(st));
   for (int s = 0; s < nsolve; ++s) h->done[s] = ctl[4 * s + 1];
   return CSADV_OK;
+}
+
+int csadv_bind_flux_tables(csadv_t *h, void *const *tables, void *stream) {
+  if (!h || !h->dev) return CSADV_E_STATE;
+  if (h->general) return fail(h, CSADV_E_STATE, "flux tables belong to the fused step");
+  const int ns = (int)h->desc.size();
+  for (int s = 0; s < ns; ++s) {
+    if (!tables || !tables[s]) continue;
+    const csadv_solve_desc &d = h->desc[s];
+    if ((uintptr_t)tables[s] % 16 != 0) return fail(h, CSADV_E_ARG, "flux tables must be 16-byte aligned");
+    if (d.ld != general_ld(d.N) || d.ldu != general_ldu(d.N))
+      return fail(h, CSADV_E_ARG, "flux tables expect ld = round_up(N+8, 4) and ldu = round_up(N+9, 4)");
+  }
+  for (int s = 0; s < ns; ++s) h->ftab[s] = tables ? tables[s] : nullptr;
+  drop_graph(h);   // the kernels of a step change with the binding
+  hipStream_t st = (hipStream_t)stream;
+  return upload_plan(h, st);
+}
+
+int csadv_refresh_winds(csadv_t *h, void *stream) {
+  if (!h || !h->dev) return CSADV_E_STATE;
+  bool any = false;
+  for (auto &d : h->desc) any = any || own_wind(d);
+  if (!any || h->mode == kWind) return CSADV_OK;
+  return wind_avg(h, (hipStream_t)stream, true);
 }
 
 int csadv_wind_init(csadv_t *h, void *stream) {
@@ -1101,7 +1175,7 @@ int enqueue_step(csadv_t *h, hipStream_t st, bool allow_prof) {
     if (rc) return rc;
     return h->dtype == CSADV_F64 ? enqueue_general_t<double>(h, st) : enqueue_general_t<float>(h, st);
   }
-  int rc = h->wind1 ? CSADV_OK : wind_avg(h, st, false);
+  int rc = wind_avg(h, st, false);
   if (rc) return rc;
   rc = step_ghosts(h, st);
   if (rc) return rc;

@@ -57,6 +57,7 @@ template <typename T> __device__ __forceinline__ T sgn(T x) { return (x > T(0)) 
 //   RECON 1 PPM-0 (CW84 eq. 1.9), 2 PPM-CW84 (monotone), 3 PPM-PL07 (eqs. 41-42), 4 PPM-L04 (B1-B4)
 template <typename T, int RECON>
 __device__ __forceinline__ void recon_edges(T m2, T m1, T c0, T p1, T p2, T &qL, T &qR) {
+#pragma clang fp contract(on)
   if constexpr (RECON == 3) {
     const T a1 = T(2.0 / 60.0), a2 = T(-13.0 / 60.0), a3 = T(47.0 / 60.0), a4 = T(27.0 / 60.0), a5 = T(-3.0 / 60.0);
     qR = a1 * m2 + a2 * m1 + a3 * c0 + a4 * p1 + a5 * p2;
@@ -191,12 +192,30 @@ struct EdgeW {
   bool up;
 };
 
+// An edge's entry in a flux table: w0, w1, w2 and, with four words, its metric-weighted Courant
+// number h (the splittings' dc = c1 - c2).  The side of the upwind cell is the lowest bit of w2:
+// that moves w2, the weight of the window's antisymmetric part (or of the far edge value), by
+// less than an ulp, where its sign or a separate wind would cost another load and compare.
+template <typename T>
+struct FluxEntry {
+  T w0, w1, w2, h;
+};
+__device__ __forceinline__ float tag_low(float v, bool b) { return __uint_as_float((__float_as_uint(v) & ~1u) | (b ? 1u : 0u)); }
+__device__ __forceinline__ double tag_low(double v, bool b) {
+  return __longlong_as_double((__double_as_longlong(v) & ~1ll) | (b ? 1ll : 0ll));
+}
+__device__ __forceinline__ bool low_tag(float v) { return __float_as_uint(v) & 1u; }
+__device__ __forceinline__ bool low_tag(double v) { return (unsigned)__double_as_longlong(v) & 1u; }
+
 // The weights of an edge with Courant number c (s as above), gA / gD the edge metrics at the edge
 // and at the upwind cell's other edge, gq its centre metric (MT-0); MT-PL07 (mt0 false) takes the
-// edge's metric gA on the whole flux.  Multiply-adds are written as fma where they fuse, so that
-// the bits do not depend on the surrounding code.
+// edge's metric gA on the whole flux.  Multiply-adds are written as fma where they fuse and the
+// compiler fuses no others (here and in the march), so that the bits do not depend on the
+// surrounding code: a solve alone and in a batch, and its weights formed in the step or read from
+// a table, agree.
 template <typename T, int RECON>
 __device__ __forceinline__ EdgeW<T> edge_weights(bool up, T c, T s, T gA, T gD, T gq, bool mt0) {
+#pragma clang fp contract(off)
   using L = Lin<RECON>;
   const T om = T(1) - s, ga = s * __builtin_elementwise_fma(T(-2), s, T(3));
   EdgeW<T> w;
@@ -226,6 +245,7 @@ __device__ __forceinline__ EdgeW<T> edge_weights(bool up, T c, T s, T gA, T gD, 
       w.w2 = -cg * (s * om);
     }
   }
+  if constexpr (!std::is_same<T, float>::value) w.w2 = tag_low(w.w2, up);   // (as a table holds it)
   return w;
 }
 
@@ -345,6 +365,32 @@ __device__ __forceinline__ void st_buf(__amdgpu_buffer_rsrc_t r, uint32_t byte_o
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, byte_off, 0, 0);
 }
 
+// Entry at byte offset off of a flux table (buffer loads: three words at once need no alignment
+// padding; the buffer covers one panel's table, under 2^32 bytes).
+typedef unsigned int csadv_u32x3 __attribute__((ext_vector_type(3)));
+typedef unsigned int csadv_u32x4 __attribute__((ext_vector_type(4)));
+template <int NW>
+__device__ __forceinline__ FluxEntry<float> ld_flux(__amdgpu_buffer_rsrc_t r, uint32_t off, float) {
+  if constexpr (NW == 3) {
+    const csadv_u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
+    return {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), 0.f};
+  } else {
+    const csadv_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+    return {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
+  }
+}
+template <int NW>
+__device__ __forceinline__ FluxEntry<double> ld_flux(__amdgpu_buffer_rsrc_t r, uint32_t off, double) {
+  typedef double f64x2 __attribute__((ext_vector_type(2)));
+  const f64x2 a = __builtin_bit_cast(f64x2, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  if constexpr (NW == 3) {
+    return {a.x, a.y, __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 16, 0)), 0.0};
+  } else {
+    const f64x2 b = __builtin_bit_cast(f64x2, __builtin_amdgcn_raw_buffer_load_b128(r, off, 16, 0));
+    return {a.x, a.y, b.x, b.y};
+  }
+}
+
 // The wind of one edge from a one-field basis W and its coefficient s at the step's time
 // (src/averaged_velocity.py:14-62 with RK1: the wind at t_n), in FP64, in one expression shared by
 // the wind kernel and the step kernel so that both give the same bits (s = 1 gives w, with a
@@ -366,11 +412,13 @@ __device__ __forceinline__ T split_update(int split, T Q, T dF, T g, T rg, T c1,
 //   AVLT: Q + dF / (2 g);  L04: Q + (dF + dc Q) / (2 g);  PL07: Q / 2 + (Q + dF) / (2 (1 - dc))
 template <typename T, int SPLIT>
 __device__ __forceinline__ T half_factor(T rg, T dc) {
+#pragma clang fp contract(off)
   if constexpr (SPLIT == 3) return T(0.5) / (T(1) - dc);
   else return T(0.5) * rg;
 }
 template <typename T, int SPLIT>
 __device__ __forceinline__ T half_step(T Q, T dF, T h, T dc) {
+#pragma clang fp contract(off)
   if constexpr (SPLIT == 1) return __builtin_elementwise_fma(h, dF, Q);
   else if constexpr (SPLIT == 2) return __builtin_elementwise_fma(h, __builtin_elementwise_fma(dc, Q, dF), Q);
   else return __builtin_elementwise_fma(h, Q + dF, T(0.5) * Q);
@@ -429,11 +477,11 @@ __device__ __forceinline__ void af_fix_cell(const Solve &S, int tr, int run, con
 // descriptor in global memory the compiler reads the words with vector loads, which warm no
 // scalar cache: the multi-solve kernel does not use it.)
 __device__ __forceinline__ int touch_solve(const Solve &S, int v) {
-  static_assert(sizeof(Solve) == 432, "one word in each 64-byte line of the descriptor");
+  static_assert(sizeof(Solve) == 448, "one word in each 64-byte line of the descriptor");
   const char *b = reinterpret_cast<const char *>(&S);
   int w[8];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) __builtin_memcpy(&w[k], b + (k < 7 ? 64 * k : 428), 4);
+  for (int k = 0; k < 8; ++k) __builtin_memcpy(&w[k], b + (k < 7 ? 64 * k : 444), 4);
   asm("" : "=s"(v) : "0"(v), "s"(w[0]), "s"(w[1]), "s"(w[2]), "s"(w[3]), "s"(w[4]), "s"(w[5]), "s"(w[6]), "s"(w[7]));
   return v;
 }

@@ -33,8 +33,8 @@ struct csadv_s {
   int split = 1;                  // splitting of every solve (its metric treatment follows)
   bool general = false;           // ET-S72 / ET-PL07: the general step
   bool mfaf = false;              // a fused-step solve with MF-AF: k_af_fix after the step kernel
-  bool wind1 = false;             // every solve RK1 with a one-field time-dependent wind: the
-                                  // step kernel forms its winds (no per-step k_wind_avg)
+  int mode = kRk1;                // FluxMode of every solve, or kMixed
+  std::vector<void *> ftab;       // the bound flux tables, one per solve (null: none)
   double *red = nullptr;          // diagnostics scratch: partials and outputs (diag_scratch_words)
   int red_tracers = 1;            // tracers the diagnostics scratch holds (the largest ntr)
   std::vector<int> done;          // host copy of the steps completed per solve (ctl[1])

@@ -140,7 +140,7 @@ std::vector<Item> wind_list(const std::vector<Solve> &solves, int &unsteady) {
   unsteady = 0;
   for (int pass = 0; pass < 2; ++pass) {
     for (int s = 0; s < (int)solves.size(); ++s) {
-      if ((solves[s].d.unsteady != 0) != (pass == 0)) continue;
+      if ((solves[s].d.unsteady && !own_wind(solves[s].d)) != (pass == 0)) continue;
       const int blocks = wind_blocks(solves[s].d.N);
       for (int pd = 0; pd < 12; ++pd)
         for (int b = 0; b < blocks; ++b) w.push_back(Item{s, pd % 6 + 8 * (pd / 6), b, 0});
@@ -162,6 +162,12 @@ int work_bytes(int N, int dtype, int64_t *bytes) {
   const WorkLayout w = work_layout(N, general_ld(N), general_ldu(N));
   const int64_t s = dtype == CSADV_F64 ? 8 : 4;
   *bytes = w.total * s + w.n_red * 8;
+  return CSADV_OK;
+}
+
+int flux_table_bytes(int N, int dtype, int split, int64_t *bytes) {
+  if (!bytes || N < 8 || N > 8192 || (dtype != CSADV_F64 && dtype != CSADV_F32) || split < 1 || split > 3) return CSADV_E_ARG;
+  *bytes = flux_elems(N, split) * (dtype == CSADV_F64 ? 8 : 4);
   return CSADV_OK;
 }
 

@@ -32,6 +32,15 @@ constexpr int kMaxTracers = 64;      // tracers per solve
 constexpr int kSegRows[] = {8, 4, 16, 32, 6, 12, 11, 5, 10, 14, 17, 23};
 constexpr int kNumTiles = sizeof(kSegRows) / sizeof(kSegRows[0]);
 
+// Where the fused step takes an edge's flux weights from:
+//   kTab        the solve's flux table (csadv_bind_flux_tables)
+//   kWind       formed in the step kernel from a one-field time-dependent wind (RK1): the FP64
+//               basis times its coefficient at the step's time (own_wind)
+//   kRk1, kRk2  formed in the step kernel from the wind arrays
+// kMixed, kMixed2: a handle of RK1 (RK2) solves that differ, each by its own mode.  In FP64 all give
+// the same bits; in FP32 a table's weights are formed in FP64 and rounded once.
+enum FluxMode : int { kRk1 = 0, kRk2 = 1, kWind = 2, kTab = 3, kMixed = 4, kMixed2 = 5 };
+
 // Device copy of one solve: the public descriptor plus derived strides.
 struct Solve {
   csadv_solve_desc d;
@@ -41,7 +50,8 @@ struct Solve {
   int64_t pstride, tstride;          // cell arrays: panel / tracer strides
   int64_t pstride_u, pstride_v;      // x-edge / y-edge arrays: panel strides
   int32_t part_per_tracer;           // partial sums per tracer (= 6 * items)
-  int32_t pad;
+  int32_t mode;                      // where its flux weights come from (FluxMode)
+  void *ftx, *fty;                   // flux tables at the x- and y-edges, or null
 };
 
 // One work item of the step kernel: (solve, panel + 8 * tracer, strip, segment); solve -1 pads.
@@ -109,6 +119,23 @@ inline int64_t general_pair_bytes(int N, int dtype) {
   return int64_t(2) * 6 * (N + 2 * NG) * general_ld(N) * (dtype == CSADV_F64 ? 8 : 4);
 }
 
+// A fused-step solve whose winds are s(t) W (RK1, one time-dependent field): the step kernel forms
+// them from the basis, where every other time-dependent solve has the wind kernel before it.
+inline bool own_wind(const csadv_solve_desc &d) {
+  return !is_general(d) && d.unsteady && d.dp == 1 && d.nbasis == 1;
+}
+
+// Flux tables: per edge the weights of its upwind flux (EdgeW, csadv_device.hpp) and, with the
+// splittings that need it, the metric-weighted Courant number: [6][M][ldu][flux_words] at the
+// x-edges, then [6][M + 1][ld][flux_words] at the y-edges.
+CSADV_HD constexpr int flux_words(int split) { return split == 1 ? 3 : 4; }
+inline int64_t flux_x_elems(int N, int split) {
+  return (int64_t)6 * (N + 2 * NG) * general_ldu(N) * flux_words(split);
+}
+inline int64_t flux_elems(int N, int split) {
+  return flux_x_elems(N, split) + (int64_t)6 * (N + 2 * NG + 1) * general_ld(N) * flux_words(split);
+}
+
 // Elements (of the state's dtype) of the work buffer the fused step needs: MF-AF keeps the
 // second pass's cube-edge fluxes, [ntr][6][4][N]; none otherwise.
 inline int64_t fused_work_elems(const csadv_solve_desc &d) {
@@ -148,12 +175,13 @@ inline int wind_blocks(int N) {
 }
 
 // The winds' work list of a multi-solve handle: (solve, panel + 8 * direction, block) of every
-// solve, the time-dependent solves first (the first `unsteady` items).
+// solve, first those whose winds are formed anew before every step (the first `unsteady` items).
 std::vector<Item> wind_list(const std::vector<Solve> &solves, int &unsteady);
 
 // Sizes of the public entry points (see include/csadv.h).
 int partials_per_tracer(int N, int tile);
 int work_bytes(int N, int dtype, int64_t *bytes);
 int tile_rows(int tile);
+int flux_table_bytes(int N, int dtype, int split, int64_t *bytes);
 
 }  // namespace csadv

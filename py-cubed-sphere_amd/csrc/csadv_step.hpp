@@ -24,7 +24,7 @@
 // src/advection_timestep.py:43)
 
 // Rows whose inputs are in flight ahead of the row being processed.
-template <typename T> constexpr int kStepPrefetch = 2;
+constexpr int kStepPrefetch = 2;
 
 // SPLIT is the splitting (1 AVLT, 2 L04, 3 PL07); the metric treatment follows from it, since
 // the valid pairs are (AVLT or L04, MT-0) and (PL07, MT-PL07) (src/discrete_operators.py:48-82).
@@ -32,10 +32,12 @@ template <typename T> constexpr int kStepPrefetch = 2;
 // the loads, wind products, metric shifts and addresses of a row serve both (the FP32 launches
 // are bound by issue), and every tracer's values are formed by the same expressions as alone,
 // which the FP32 units fuse per expression, so the bits are the same.
-template <typename T, int RECON, bool RK2, int SPLIT, bool WIND = false, bool XPULL = false, int NT = 1>
+template <typename T, int RECON, int MODE, int SPLIT, bool XPULL = false, int NT = 1>
 struct March {
+  static constexpr bool TAB = MODE == kTab, WIND = MODE == kWind, RK2 = MODE == kRk2;
+  static constexpr int NW = flux_words(SPLIT);     // words of a flux-table entry
   static constexpr int split = SPLIT;
-  static constexpr int PF = kStepPrefetch<T>;
+  static constexpr int PF = kStepPrefetch;
   // Two arrangements of the per-row values, by precision (measured):
   //  * EXACT (FP64, where a single solve leaves about two wavefronts per SIMD, so each
   //    wavefront's waits are exposed): every per-row value, loaded or computed, sits in a ring
@@ -64,10 +66,9 @@ struct March {
   static constexpr int sl(int K, int j) { return ((K + j) % RD + RD) % RD; }
   // ---- inputs (per wavefront; Q, Qa per tracer)
   const T *Q[NT], *Qa[NT], *U, *US, *V, *VS, *gc, *gu, *gv, *rgc, *gfix;
-  // WIND: the winds of the step are formed here from the one-field FP64 basis (WU, WV) and its
-  // coefficient ws at the step's time, as k_wind_avg forms them for RK1, instead of read
-  const double *WU, *WV;
+  const double *WU, *WV;                // kWind
   double ws;
+  __amdgpu_buffer_rsrc_t ftx, fty;      // kTab: this panel's flux tables
   T *Qo[NT];                       // the output panel of each tracer ([M][ld])
   __amdgpu_buffer_rsrc_t qo_buf;   // the same, for the stores of the EXACT arrangement
   int ld, ldu, M, iend, x, xc, xe, tj, ylast;
@@ -94,24 +95,34 @@ struct March {
   //   (per tracer: qr, qar, qw, xw, sw, the flux carries and the partial sum)
   T qr[NT][RS], gfr[RS], qar[NT][RS], ur[RS], usr[RS], gur[RS], vr[RS], vsr[RS];
   T qw[NT][RD], xw[NT][RD], sw[NT][RD], gcw[RD], rgw[RD], gvr[RD];
-  T x0[RD], x1[RD], x2[RD];
+  T x0[RD], x1[RD], x2[RD], y0[RS], y1[RS], y2[RS];
   bool xup[RD];
   T g1prev[NT], g2prev[NT], hyprev;
   Cell<T> pa[NT], pb[NT];          // row y-4 as the left cell of edge y-3: Q, Qx
   double part[NT];
 
-  // Inputs of row y into ring slot SLOT.  SPEC: also read Q from the other state buffer (Qa),
-  // for the rows requested before the step counter has arrived.
-  template <bool SPEC, int SLOT>
+  // Inputs of row y into ring slot SLOT.  J: the row's offset from the item's first row where it is
+  // known at compile time (the first rows: no y-edge is read before the column stage needs it,
+  // kYFrom for its flux weights and two rows earlier for the edge metric), else kSteady.  SPEC:
+  // also read Q from the other state buffer (Qa), for the rows requested before the step counter
+  // has arrived.  Rows past the item's last are requested as that row again (in cache).
+  static constexpr int kYFrom = 6, kSteady = 64;
+  template <bool SPEC, int SLOT, int J = kSteady>
   __device__ __forceinline__ void load(int y) {
-    const int yc = min(y, M - 1);
+    const int yc = min(y, ylast);
     const uint32_t o = (uint32_t)(yc * ld + xc), ou = (uint32_t)(yc * ldu + xe);
     constexpr int SS = SLOT % RS;          // state slot
-    if constexpr (WIND) ur[SS] = T(wind_of_basis(ws, ld_at(WU, ou)));
-    else ur[SS] = ld_at(U, ou);
-    if constexpr (RK2) usr[SS] = ld_at(US, ou);
-    gur[SS] = ld_at(gu, ou);
-    gcw[SLOT] = ld_at(gc, o);
+    if constexpr (TAB) {
+      const FluxEntry<T> f = ld_flux<NW>(ftx, ou * (uint32_t)(NW * sizeof(T)), T(0));
+      x0[SLOT] = f.w0; x1[SLOT] = f.w1; x2[SLOT] = f.w2;
+      if constexpr (NW == 4) ur[SS] = f.h;
+    } else {
+      if constexpr (WIND) ur[SS] = T(wind_of_basis(ws, ld_at(WU, ou)));
+      else ur[SS] = ld_at(U, ou);
+      if constexpr (RK2) usr[SS] = ld_at(US, ou);
+      gur[SS] = ld_at(gu, ou);
+      gcw[SLOT] = ld_at(gc, o);
+    }
     rgw[SLOT] = ld_at(rgc, o);
     gfr[SS] = ld_at(gfix, o);
     // Q of every lane, at the clamped row and column (rows past ylast are requested too): no
@@ -132,11 +143,20 @@ struct March {
         }
       }
     }
-    const int ec = min(max(y - 3, 0), M - 1);
-    if constexpr (WIND) vr[SS] = T(wind_of_basis(ws, ld_at(WV, (uint32_t)(ec * ld + xc))));
-    else vr[SS] = ld_at(V, (uint32_t)(ec * ld + xc));
-    if constexpr (RK2) vsr[SS] = ld_at(VS, (uint32_t)(ec * ld + xc));
-    gvr[SLOT] = ld_at(gv, (uint32_t)((ec + 1) * ld + xc));
+    if constexpr (J < kYFrom - 2) return;
+    const int ec = yc - 3;               // a y-edge of the item from its fourth row on
+    if constexpr (TAB) {
+      if constexpr (J < kYFrom) return;
+      const FluxEntry<T> f = ld_flux<NW>(fty, (uint32_t)(ec * ld + xc) * (uint32_t)(NW * sizeof(T)), T(0));
+      y0[SS] = f.w0; y1[SS] = f.w1; y2[SS] = f.w2;
+      if constexpr (NW == 4) vr[SS] = f.h;
+    } else {
+      gvr[SLOT] = ld_at(gv, (uint32_t)((ec + 1) * ld + xc));
+      if constexpr (J < kYFrom) return;
+      if constexpr (WIND) vr[SS] = T(wind_of_basis(ws, ld_at(WV, (uint32_t)(ec * ld + xc))));
+      else vr[SS] = ld_at(V, (uint32_t)(ec * ld + xc));
+      if constexpr (RK2) vsr[SS] = ld_at(VS, (uint32_t)(ec * ld + xc));
+    }
   }
 
   // whether row y at this lane's column is within the stencils' reach (the columns and rows of
@@ -150,6 +170,7 @@ struct March {
   // outside the stencils' reach hold 0 + C gfix, which no stored cell reads.
   // (with no correction total, cf = 0 and q + 0 gfix = q: no branch on the mass fixer)
   __device__ __forceinline__ T corrected(T raw, T gf, int t) const {
+#pragma clang fp contract(off)
     if constexpr (std::is_same<T, float>::value) return __builtin_elementwise_fma(T(cf[t]), gf, raw + off[t]);
     else return __builtin_elementwise_fma(T(cf[t]), gf, raw);
   }
@@ -159,8 +180,9 @@ struct March {
   // (STAGE >= 1), fluxes through y-edge y-3 from tj+3 on (>= 2), the update of row y-4 from
   // tj+4 on (3).  The first seven rows are peeled with their stage; every later row is 3, so
   // the loop carries no per-row test.
-  template <int K, int STAGE>
+  template <int K, int STAGE, int J>
   __device__ __forceinline__ void body(const int y) {
+#pragma clang fp contract(off)
     // slots of rows y, y-5 .. y-1, and of row y in the state rings
     constexpr int s0 = sl(K, 0), s1 = sl(K, -5), s2 = sl(K, -4), s3 = sl(K, -3), s4 = sl(K, -2), s5 = sl(K, -1);
     constexpr int ss = s0 % RS;
@@ -181,12 +203,18 @@ struct March {
         b[t] = cell_of<T, RECON>(xw[t][s1], xw[t][s2], xw[t][s3], xw[t][s4], xw[t][s5]);
       }
       if constexpr (STAGE >= 2) {
-        const T cy = vr[ss] * dtdy;
-        const bool vup = (RK2 ? vsr[ss] : vr[ss]) >= T(0);
-        const EdgeW<T> wy = edge_weights<T, RECON>(vup, cy, RK2 ? (vup ? cy : -cy) : fabs_t(cy), gv0, vup ? gvm1 : gvp1,
-                                                   vup ? gcw[s2] : gcw[s3], mt0);
+        EdgeW<T> wy;
         T hy = T(0);
-        if constexpr (split != 1) hy = gv0 * cy;
+        if constexpr (TAB) {
+          wy = EdgeW<T>{y0[ss], y1[ss], y2[ss], low_tag(y2[ss])};
+          if constexpr (split != 1) hy = vr[ss];
+        } else {
+          const T cy = vr[ss] * dtdy;
+          const bool vup = (RK2 ? vsr[ss] : vr[ss]) >= T(0);
+          wy = edge_weights<T, RECON>(vup, cy, RK2 ? (vup ? cy : -cy) : fabs_t(cy), gv0, vup ? gvm1 : gvp1,
+                                      vup ? gcw[s2] : gcw[s3], mt0);
+          if constexpr (split != 1) hy = gv0 * cy;
+        }
         T g1[NT], g2[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
@@ -196,7 +224,7 @@ struct March {
         if constexpr (STAGE >= 3) {
           const T rg = rgw[s2];                // row y-4
           const T h = half_factor<T, SPLIT>(rg, hy - hyprev);
-          const EdgeW<T> wx{x0[s2], x1[s2], x2[s2], xup[s2]};
+          const EdgeW<T> wx{x0[s2], x1[s2], x2[s2], TAB ? low_tag(x2[s2]) : xup[s2]};
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
             const T dG1 = g1prev[t] - g1[t];
@@ -242,17 +270,22 @@ struct March {
     // last parabola row is ylast-3, whose window ends at ylast-1).  FP32, bound by issue, skips
     // it by a wave-uniform branch (2-3% of the launch).
     if (!std::is_same<T, float>::value || STAGE < 3 || y < ylast) {
-      const T u = ur[ss], gu0 = gur[ss], gc0 = gcw[s0], cx = u * dtdx;
-      const bool up = (RK2 ? usr[ss] : u) >= T(0);
-      // (the lane shifts before the selects: every lane takes part in them)
-      const T gul = from_left(gu0), gur1 = from_right(gu0), gcl = from_left(gc0);
-      const EdgeW<T> wx = edge_weights<T, RECON>(up, cx, RK2 ? (up ? cx : -cx) : fabs_t(cx), gu0, up ? gul : gur1,
-                                                 up ? gcl : gc0, mt0);
-      x0[s0] = wx.w0; x1[s0] = wx.w1; x2[s0] = wx.w2; xup[s0] = up;
+      EdgeW<T> wx;
       T dh = T(0);
-      if constexpr (split != 1) {
-        const T hx0 = gu0 * cx;
-        dh = from_right(hx0) - hx0;
+      if constexpr (TAB) {
+        wx = EdgeW<T>{x0[s0], x1[s0], x2[s0], low_tag(x2[s0])};
+        if constexpr (split != 1) dh = from_right(ur[ss]) - ur[ss];
+      } else {
+        const T u = ur[ss], gu0 = gur[ss], gc0 = gcw[s0], cx = u * dtdx;
+        const bool up = (RK2 ? usr[ss] : u) >= T(0);
+        // (the lane shifts before the selects: every lane takes part in them)
+        const T gul = from_left(gu0), gur1 = from_right(gu0), gcl = from_left(gc0);
+        wx = edge_weights<T, RECON>(up, cx, RK2 ? (up ? cx : -cx) : fabs_t(cx), gu0, up ? gul : gur1, up ? gcl : gc0, mt0);
+        x0[s0] = wx.w0; x1[s0] = wx.w1; x2[s0] = wx.w2; xup[s0] = up;
+        if constexpr (split != 1) {
+          const T hx0 = gu0 * cx;
+          dh = from_right(hx0) - hx0;
+        }
       }
       const T h = half_factor<T, SPLIT>(rgw[s0], dh);
 #pragma unroll
@@ -269,8 +302,7 @@ struct March {
       qw[t][s0] = q[t];
       sw[t][s0] = raw[t];
     }
-    // rows past ylast are read in bounds (clamped rows, masked Q) and never used
-    load<false, sl(K, PF)>(y + PF);
+    load<false, sl(K, PF), J == kSteady ? kSteady : J + PF>(y + PF);
     // EXACT: the output row's store, after the loads and issued by every lane (the first rows,
     // which have no output row yet, issue it too, dropped)
     if constexpr (EXACT)
@@ -279,7 +311,7 @@ struct March {
 
   template <int... J>
   __device__ __forceinline__ void first_rows(std::integer_sequence<int, J...>) {
-    (load<true, J>(tj - 3 + J), ...);
+    (load<true, J, J>(tj - 3 + J), ...);
   }
 
   // The first PF rows' inputs, requested before the step counter is known: Q from both state
@@ -291,7 +323,7 @@ struct March {
       xup[k] = false;
     }
 #pragma unroll
-    for (int k = 0; k < RS; ++k) gfr[k] = ur[k] = usr[k] = gur[k] = vr[k] = vsr[k] = T(0);
+    for (int k = 0; k < RS; ++k) gfr[k] = ur[k] = usr[k] = gur[k] = vr[k] = vsr[k] = y0[k] = y1[k] = y2[k] = T(0);
     hyprev = T(0);   // gv is complete from y = tj-1 on; the column stage starts at tj+2
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -320,7 +352,7 @@ struct March {
   // row y0 + K0 + j in phase (K0 + j) % RD
   template <int K0, int STAGE, int J>
   __device__ __forceinline__ void row(int y) {
-    body<(K0 + J) % RD, STAGE>(y + J);
+    body<(K0 + J) % RD, STAGE, K0 == 0 ? J : kSteady>(y + J);
   }
   template <int K0, int... J>
   __device__ __forceinline__ void full_rows(int y, std::integer_sequence<int, J...>) {
@@ -343,9 +375,10 @@ struct March {
 };
 
 // One work item: NT tracers tr, tr+1, .. of one (panel, strip, segment).
-template <typename T, int RECON, bool RK2, int SPLIT, bool WIND, bool XPULL, int NT = 1>
+template <typename T, int RECON, int MODE, int SPLIT, bool XPULL, int NT = 1>
 __device__ __forceinline__ void step_item(const Solve &S, const int4 wk) {
-  using Mt = March<T, RECON, RK2, SPLIT, WIND, XPULL, NT>;
+  using Mt = March<T, RECON, MODE, SPLIT, XPULL, NT>;
+  constexpr bool RK2 = MODE == kRk2;
   const int lane = threadIdx.x;
   const csadv_solve_desc &D = S.d;
   const int p = wk.y & 7, tr = wk.y >> 3;    // panel, (first) tracer
@@ -397,7 +430,12 @@ __device__ __forceinline__ void step_item(const Solve &S, const int4 wk) {
     m.Qa[t] = reinterpret_cast<const T *>(D.q1) + off[t];
   }
   int step;
-  if constexpr (WIND) {
+  if constexpr (MODE == kTab) {
+    constexpr int64_t entry = flux_words(SPLIT) * sizeof(T);
+    m.ftx = buffer_of(static_cast<char *>(S.ftx) + p * S.pstride_u * entry, (uint32_t)(S.pstride_u * entry));
+    m.fty = buffer_of(static_cast<char *>(S.fty) + p * S.pstride_v * entry, (uint32_t)(S.pstride_v * entry));
+  }
+  if constexpr (MODE == kWind) {
     // the winds of the first rows need the step's coefficient: the step counter comes first
     step = D.ctl[2];
     const int row = min(max(step, 0), D.max_steps - 1);   // as k_wind_avg (one basis field)
@@ -451,21 +489,31 @@ template <typename T> constexpr int kStepGroup = std::is_same<T, float>::value ?
 
 // One item of NT = kStepGroup<T> tracers, or of one where the solve has no second tracer left
 // (a wave-uniform choice).
-template <typename T, int RECON, bool RK2, int SPLIT, bool WIND, bool XPULL>
+template <typename T, int RECON, int MODE, int SPLIT, bool XPULL>
 __device__ __forceinline__ void step_group(const Solve &S, const int4 wk) {
-  if constexpr (kStepGroup<T> == 2) {
-    if ((wk.y >> 3) + 1 < S.d.ntr) step_item<T, RECON, RK2, SPLIT, WIND, XPULL, 2>(S, wk);
-    else step_item<T, RECON, RK2, SPLIT, WIND, XPULL, 1>(S, wk);
+  if constexpr (MODE == kMixed) {
+    if (S.mode == kTab) step_group<T, RECON, kTab, SPLIT, XPULL>(S, wk);
+    else if (S.mode == kWind) step_group<T, RECON, kWind, SPLIT, XPULL>(S, wk);
+    else step_group<T, RECON, kRk1, SPLIT, XPULL>(S, wk);
+  } else if constexpr (MODE == kMixed2) {
+    if (S.mode == kTab) step_group<T, RECON, kTab, SPLIT, XPULL>(S, wk);
+    else step_group<T, RECON, kRk2, SPLIT, XPULL>(S, wk);
+  } else if constexpr (kStepGroup<T> == 2) {
+    if ((wk.y >> 3) + 1 < S.d.ntr) step_item<T, RECON, MODE, SPLIT, XPULL, 2>(S, wk);
+    else step_item<T, RECON, MODE, SPLIT, XPULL, 1>(S, wk);
   } else {
-    step_item<T, RECON, RK2, SPLIT, WIND, XPULL, 1>(S, wk);
+    step_item<T, RECON, MODE, SPLIT, XPULL, 1>(S, wk);
   }
 }
 
-template <typename T, int RECON, bool RK2, int SPLIT, bool WIND>
-__global__ __launch_bounds__(WAVE) void k_step(const Solve *__restrict__ solves, const int4 *__restrict__ work) {
+// Wavefronts per SIMD the registers must leave room for: the FP64 RK2 march would otherwise take a
+// few too many for two.
+template <typename T> constexpr int kMinWaves = std::is_same<T, float>::value ? 1 : 2;
+template <typename T, int RECON, int MODE, int SPLIT>
+__global__ __launch_bounds__(WAVE, kMinWaves<T>) void k_step(const Solve *__restrict__ solves, const int4 *__restrict__ work) {
   const int4 wk = work[blockIdx.x];
   if (wk.x < 0) return;              // padding item of the XCD-banded work list
-  step_group<T, RECON, RK2, SPLIT, WIND, false>(solves[wk.x], wk);
+  step_group<T, RECON, MODE, SPLIT, false>(solves[wk.x], wk);
 }
 
 // Work item b of a single-solve handle, computed instead of read: the list the host builds
@@ -486,27 +534,33 @@ __device__ __forceinline__ bool single_item(const Solve &S, int b, int4 &wk) {
 // computed, so the first loads of a wavefront depend on nothing but the arguments.
 // FP32 takes its x windows through the crossbar (measured 3% faster at N=768 with 4 tracers);
 // FP64 and the multi-solve kernel keep the DPP shifts (measured 0.5-4% slower with the crossbar).
-template <typename T, int RECON, bool RK2, int SPLIT, bool WIND>
-__global__ __launch_bounds__(WAVE) void k_step1(const Solve one) {
+template <typename T, int RECON, int MODE, int SPLIT>
+__global__ __launch_bounds__(WAVE, kMinWaves<T>) void k_step1(const Solve one) {
   int4 wk;
   if (!single_item(one, touch_solve(one, blockIdx.x), wk)) return;
-  step_item<T, RECON, RK2, SPLIT, WIND, std::is_same<T, float>::value>(one, wk);
+  step_item<T, RECON, MODE, SPLIT, std::is_same<T, float>::value>(one, wk);
+}
+
+template <typename T, int R, int MODE, int SP>
+void launch_step_m(csadv_t *h, hipStream_t st) {
+  if constexpr (MODE < kMixed) {
+    if (h->host.size() == 1) {
+      hipLaunchKernelGGL((k_step1<T, R, MODE, SP>), dim3(h->nwork), dim3(WAVE), 0, st, h->host[0]);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_step<T, R, MODE, SP>), dim3(h->nwork), dim3(WAVE), 0, st, h->dev, h->work);
 }
 
 template <typename T, int R, int SP>
 hipError_t launch_step_s(csadv_t *h, hipStream_t st) {
-  const bool one = h->host.size() == 1;
-  if (h->wind1) {                    // RK1 only
-    if (one) hipLaunchKernelGGL((k_step1<T, R, false, SP, true>), dim3(h->nwork), dim3(WAVE), 0, st, h->host[0]);
-    else hipLaunchKernelGGL((k_step<T, R, false, SP, true>), dim3(h->nwork), dim3(WAVE), 0, st, h->dev, h->work);
-    return hipGetLastError();
-  }
-  if (h->rk2) {
-    if (one) hipLaunchKernelGGL((k_step1<T, R, true, SP, false>), dim3(h->nwork), dim3(WAVE), 0, st, h->host[0]);
-    else hipLaunchKernelGGL((k_step<T, R, true, SP, false>), dim3(h->nwork), dim3(WAVE), 0, st, h->dev, h->work);
-  } else {
-    if (one) hipLaunchKernelGGL((k_step1<T, R, false, SP, false>), dim3(h->nwork), dim3(WAVE), 0, st, h->host[0]);
-    else hipLaunchKernelGGL((k_step<T, R, false, SP, false>), dim3(h->nwork), dim3(WAVE), 0, st, h->dev, h->work);
+  switch (h->mode) {
+    case kMixed: launch_step_m<T, R, kMixed, SP>(h, st); break;
+    case kMixed2: launch_step_m<T, R, kMixed2, SP>(h, st); break;
+    case kWind: launch_step_m<T, R, kWind, SP>(h, st); break;
+    case kTab: launch_step_m<T, R, kTab, SP>(h, st); break;
+    case kRk2: launch_step_m<T, R, kRk2, SP>(h, st); break;
+    default: launch_step_m<T, R, kRk1, SP>(h, st);
   }
   return hipGetLastError();
 }

@@ -16,6 +16,7 @@ _ERRORS = {-1: "invalid argument", -2: "HIP runtime error", -3: "call out of ord
 # exported symbols, in declaration order of include/csadv.h
 SYMBOLS = (
     "csadv_create", "csadv_partials_per_tracer", "csadv_work_bytes", "csadv_tile_rows", "csadv_update", "csadv_wind_init",
+    "csadv_flux_table_bytes", "csadv_bind_flux_tables", "csadv_refresh_winds",
     "csadv_ghost_fill", "csadv_step", "csadv_set_graph", "csadv_finalize", "csadv_mass", "csadv_norms",
     "csadv_diagnostics", "csadv_diagnostics_noalloc", "csadv_status",
     "csadv_current", "csadv_profile", "csadv_profile_read", "csadv_time_step_kernel", "csadv_time_step_kernel_rotating", "csadv_remap_latlon", "csadv_last_error", "csadv_destroy",
@@ -69,6 +70,9 @@ def load():
     lib.csadv_work_bytes.argtypes = [i32, i32, ctypes.POINTER(ctypes.c_int64)]
     lib.csadv_update.argtypes = [vp, ctypes.POINTER(SolveDesc), i32, vp]
     lib.csadv_wind_init.argtypes = [vp, vp]
+    lib.csadv_flux_table_bytes.argtypes = [i32, i32, i32, ctypes.POINTER(ctypes.c_int64)]
+    lib.csadv_bind_flux_tables.argtypes = [vp, ctypes.POINTER(vp), vp]
+    lib.csadv_refresh_winds.argtypes = [vp, vp]
     lib.csadv_ghost_fill.argtypes = [vp, vp]
     lib.csadv_step.argtypes = [vp, i32, vp]
     lib.csadv_set_graph.argtypes = [vp, i32]

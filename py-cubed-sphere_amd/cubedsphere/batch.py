@@ -48,7 +48,7 @@ class Batch:
         self._open(self.members)
         return self
 
-    def _create(self, members):
+    def _create(self, members, fill=False):
         descs = (_lib.SolveDesc * len(members))(*[m.desc() for m in members])
         h = ctypes.c_void_p()
         rc = self.lib.csadv_create(descs, len(members), 0, ctypes.byref(h))
@@ -56,13 +56,18 @@ class Batch:
             msg = self.lib.csadv_last_error(h).decode()
             self.lib.csadv_destroy(h)
             raise _lib.CsadvError("csadv_create: %s" % msg)
+        try:
+            Advection.bind_flux_tables(self.lib, h, members, self._stream(), fill)
+        except _lib.CsadvError:
+            self.lib.csadv_destroy(h)
+            raise
         return h
 
     def _open(self, fresh):
         """Prepare the winds of the fresh members (on a handle of their own, so members that
         are already running are not touched), then one handle over every member."""
         if fresh:
-            h = self._create(fresh)
+            h = self._create(fresh, fill=True)
             rc = self.lib.csadv_wind_init(h, self._stream())
             msg = self.lib.csadv_last_error(h).decode() if rc else ""
             self.lib.csadv_destroy(h)
