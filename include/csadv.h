@@ -141,7 +141,7 @@ int csadv_update(csadv_t *h, const csadv_solve_desc *solves, int32_t nsolve, voi
  * (src/averaged_velocity.py:14-62).  Call once after the basis interiors are written. */
 int csadv_wind_init(csadv_t *h, void *stream);
 
-/* Flux tables (fused step): the weights of the upwind fluxes depend on the winds and the metric
+/* Flux tables (fused step, FP64): the weights of the upwind fluxes depend on the winds and the metric
  * only, so a solve whose winds are steady (or are recombined by the wind kernel) can keep them
  * in a caller-owned device buffer instead of forming them in every step.  csadv_flux_table_bytes
  * gives its size; csadv_bind_flux_tables hands one buffer per solve to the handle (tables[s], 16-
@@ -150,7 +150,7 @@ int csadv_wind_init(csadv_t *h, void *stream);
  * them.  A filled table may be bound to any later handle over the same solve (same dt, dx, options
  * and winds) without another csadv_wind_init.  A solve with RK1 and a one-field time-dependent wind
  * uses none (the step forms its winds).  csadv_update keeps the binding.  No counterpart in the reference. */
-int csadv_flux_table_bytes(int32_t N, int32_t dtype, int32_t split, int64_t *bytes);
+int csadv_flux_table_bytes(int32_t N, int32_t split, int64_t *bytes);
 int csadv_bind_flux_tables(csadv_t *h, void *const *tables, void *stream);
 
 /* uavg / vavg of the next step for the solves whose winds the step kernel forms (RK1, one time-

@@ -152,16 +152,6 @@ __device__ double partial_sum(const double *P, int n, double *red) {
   return block_sum_fixed(acc, red);
 }
 
-// Mass-fixer correction total C after `steps` steps, from the stored totals c0 / c1 (slots of
-// even / odd steps) and the partials' sum: with the partials of the last step pending,
-// C = C(steps - 1) + dt m0 / a2, m0 = sum of div g over the interior
-// (src/discrete_operators.py:98-101); otherwise C is the stored total of this step.
-__device__ __forceinline__ double corr_total(double dt, double a2, double c0, double c1, double sum, int pending,
-                                             int steps) {
-  const double held = (steps & 1) ? c1 : c0, prev = (steps & 1) ? c0 : c1;
-  return pending ? prev + dt * sum / a2 : held;
-}
-
 // blk: the block of BLOCK ghost cells, or -1 for the tracer's correction-total block; tr: tracer.
 template <typename T>
 __device__ __forceinline__ void ghost_cells(const Solve &S, double *red, int blk, int tr) {
@@ -245,16 +235,13 @@ __device__ __forceinline__ void ghost_cells(const Solve &S, double *red, int blk
   if (active) {
     if (strip) {
       const T v0 = Qt[s16[0]], v1 = Qt[s16[1]], v2 = Qt[s16[2]], v3 = Qt[s16[3]];
-      acc += (double)v0 * w16[0];
-      acc += (double)v1 * w16[1];
-      acc += (double)v2 * w16[2];
-      acc += (double)v3 * w16[3];
+      acc = strip_sum((double)v0, (double)v1, (double)v2, (double)v3, w16[0], w16[1], w16[2], w16[3]);
     } else {
       T v[16];
 #pragma unroll
       for (int l = 0; l < 16; ++l) v[l] = Qt[s16[l]];
 #pragma unroll
-      for (int l = 0; l < 16; ++l) acc += (double)v[l] * w16[l];
+      for (int l = 0; l < 16; ++l) acc = fma((double)v[l], w16[l], acc);
     }
     Qt[tgt] = (T)acc;
   }
@@ -344,6 +331,72 @@ __global__ __launch_bounds__(BLOCK) void k_af_fix(const Solve *solves) {
   const int run = D.ctl[2];                 // the step k_ghost started (< 0: the solve is halted)
   if (run < 0 || (D.stop > 0 && run >= D.stop)) return;
   af_fix_cell<T>(S, tr, run, reinterpret_cast<const T *>(D.work) + (int64_t)tr * 24 * D.N, blockIdx.x * BLOCK + threadIdx.x);
+}
+
+// A handle of one solve whose steps fill their own ghosts: step k of the running sequence (the
+// completed steps, ctl[1], stand still until its end).  grid: x = boundary cells, y = tracer.
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void k_af_fix1(const Solve one, int k) {
+  const csadv_solve_desc &D = one.d;
+  const int tr = blockIdx.y, run = D.ctl[1] + k;
+  if (D.ctl[0] || (D.stop > 0 && run >= D.stop)) return;
+  af_fix_cell<T>(one, tr, run, reinterpret_cast<const T *>(D.work) + (int64_t)tr * 24 * D.N, blockIdx.x * BLOCK + threadIdx.x);
+}
+
+// End of a sequence of n steps that filled their own ghosts: the last executed step's mass-fixer
+// partials (in b0 or b1, by its place in the sequence) go into the correction total, and the step
+// counter takes all executed steps at once.  One block.
+__global__ __launch_bounds__(BLOCK) void k_advance(const Solve one, int n, const double *b0, const double *b1) {
+  __shared__ double red[BLOCK];
+  const csadv_solve_desc &D = one.d;
+  const int steps = D.ctl[1], halted = D.ctl[0];
+  const int m = halted ? 0 : (D.stop > 0 ? min(n, D.stop - steps) : n);
+  __syncthreads();                     // every thread has read the counter
+  if (m <= 0) return;
+  if (D.mf == 3) {
+    const double *P = (m - 1) & 1 ? b1 : b0;
+    for (int tr = 0; tr < D.ntr; ++tr) {
+      const double c0 = D.corr[tr], c1 = D.corr[D.ntr + tr];
+      const double sum = partial_sum(P + (int64_t)tr * one.part_per_tracer, one.part_per_tracer, red);
+      if (threadIdx.x == 0)
+        D.corr[((steps + m) & 1) * D.ntr + tr] = corr_total(D.dt, D.a2, c0, c1, sum, 1, steps + m);
+    }
+  }
+  if (threadIdx.x == 0) {
+    D.ctl[1] = steps + m;
+    D.ctl[2] = steps + m - 1;
+    D.ctl[3] = 0;
+  }
+}
+
+// Whether the ghost recipes are those of the Lagrange tables in the order the self-filling step
+// reads them (ok stays 1): strips by (panel, side), the depth slowest where the source strip runs
+// along x and fastest elsewhere; corners by (panel, E / W, depth, row).
+__global__ __launch_bounds__(BLOCK) void k_check_recipes(const Solve one, int32_t *ok) {
+  const csadv_solve_desc &D = one.d;
+  const int N = D.N, M = one.M, ld = D.ld, n = 72 * N + 216;
+  for (int t = blockIdx.x * BLOCK + threadIdx.x; t < n; t += gridDim.x * BLOCK) {
+    bool same = true;
+    int i, j;
+    if (t < 72 * N) {
+      const int ps = t / (3 * N), r = t - ps * 3 * N, p = ps >> 2, side = ps & 3;
+      const int32_t *o = D.orient + ps * 7;
+      const int d = o[3] != 0 ? r / N : r % 3, k = NG + (o[3] != 0 ? r % N : r / 3);
+      ghost_target(side, d, k, N, i, j);
+      same = D.strip_tgt[t] == p * (int)one.pstride + j * ld + i;
+      for (int l = 0; l < 4; ++l) {
+        int q, si, sj;
+        halo_src(o, d, D.lagk[d * M + k] + l, q, si, sj);
+        same = same && D.strip_src[4 * (int64_t)t + l] == q * (int)one.pstride + sj * ld + si &&
+               D.strip_w[4 * (int64_t)t + l] == D.lagw[((int64_t)d * M + k) * 4 + l];
+      }
+    } else {
+      const int c = t - 72 * N, m = c % 6, d = (c / 6) % 3, side = (c / 18) & 1, p = c / 36;
+      ghost_target(side, d, corner_row(m, N), N, i, j);
+      same = D.corner_tgt[c] == p * (int)one.pstride + j * ld + i;
+    }
+    if (!same) *ok = 0;
+  }
 }
 
 // ------------------------------------------------------------------ lat-lon output remap
@@ -532,13 +585,12 @@ __device__ __forceinline__ double wind_comb(const double *W, int64_t bs, const d
 }
 
 // The flux-table entry of an edge (x: edge e of row r; y: edge r of column e) with upwind-side
-// wind u and averaged wind avg, formed in FP64 and rounded once.
-template <typename T>
-__device__ __forceinline__ FluxEntry<T> flux_entry(const csadv_solve_desc &D, bool xdir, int64_t r, int64_t e, double u,
-                                                   double avg) {
+// wind u and averaged wind avg: what the step would form there.
+__device__ __forceinline__ FluxEntry<double> flux_entry(const csadv_solve_desc &D, bool xdir, int64_t r, int64_t e,
+                                                        double u, double avg) {
 #pragma clang fp contract(off)
   const bool up = u >= 0.0, mt0 = D.split != 3;
-  const T *gm = reinterpret_cast<const T *>(xdir ? D.gu : D.gv);
+  const double *gm = reinterpret_cast<const double *>(xdir ? D.gu : D.gv);
   const int64_t row = xdir ? D.ldu : D.ld, step = xdir ? 1 : D.ld, o = r * row + e, oc = r * D.ld + e;
   const double gA = gm[o], gD = gm[up ? o - step : o + step], gq = D.gc64[up ? oc - step : oc];
   const double c = avg * (D.dt / (xdir ? D.dx : D.dy)), s = up ? c : -c;
@@ -546,18 +598,18 @@ __device__ __forceinline__ FluxEntry<T> flux_entry(const csadv_solve_desc &D, bo
   if (D.recon == 3) w = edge_weights<double, 3>(up, c, s, gA, gD, gq, mt0);
   else if (D.recon == 1) w = edge_weights<double, 1>(up, c, s, gA, gD, gq, mt0);
   else w = edge_weights<double, 2>(up, c, s, gA, gD, gq, mt0);
-  return {(T)w.w0, (T)w.w1, tag_low((T)w.w2, up), (T)(gA * c)};
+  return {w.w0, w.w1, w.w2, gA * c};
 }
 
 // Block blk of the x-edges (dir 0) or y-edges (dir 1) of panel p.
 template <typename T, int KB>
-__device__ __forceinline__ void wind_edges(const Solve &S, int p, int dir, int blk) {
+__device__ __forceinline__ void wind_edges(const Solve &S, int p, int dir, int blk, int steps) {
   const csadv_solve_desc &D = S.d;
   const int N = D.N, M = S.M, ld = D.ld, ldu = D.ldu, K = KB ? KB : D.nbasis;
   const bool xdir = dir == 0, rk2 = D.dp == 2;
   const int64_t ps = xdir ? S.pstride_u : S.pstride_v, bs = 6 * ps, step = xdir ? 1 : ld;
   const double *W = (xdir ? D.wbu : D.wbv) + p * ps;
-  const int row = D.unsteady ? min(D.ctl[1], D.max_steps - 1) : 0;   // steps completed
+  const int row = D.unsteady ? min(steps, D.max_steps - 1) : 0;
   const double *s1 = D.coef + (int64_t)row * 2 * K;   // coefficients at t_{n-1}
   const double *s0 = s1 + K;                          // at t_{n-2}
   // x-edges as [row 0 .. M-1][edge i0 .. iend], y-edges as [edge i0 .. iend][column 0 .. M-1]
@@ -592,11 +644,12 @@ __device__ __forceinline__ void wind_edges(const Solve &S, int p, int dir, int b
     if (first + k * BLOCK >= total) continue;
     ua[off[k]] = (T)avg[k];
     if (us) us[p * ps + off[k]] = (T)u[k];
-    if (S.ftx) {
+    if constexpr (!std::is_same<T, float>::value) {
+      if (!S.ftx) continue;
       const int nw = flux_words(D.split), row = xdir ? ldu : ld;
       const int64_t r = off[k] / row, e = off[k] - r * row;
-      const FluxEntry<T> f = flux_entry<T>(D, xdir, r, e, u[k], avg[k]);
-      T *o = reinterpret_cast<T *>(xdir ? S.ftx : S.fty) + (p * ps + off[k]) * nw;
+      const FluxEntry<double> f = flux_entry(D, xdir, r, e, u[k], avg[k]);
+      double *o = static_cast<double *>(xdir ? S.ftx : S.fty) + (p * ps + off[k]) * nw;
       o[0] = f.w0; o[1] = f.w1; o[2] = f.w2;
       if (nw == 4) o[3] = f.h;
     }
@@ -604,12 +657,13 @@ __device__ __forceinline__ void wind_edges(const Solve &S, int p, int dir, int b
 }
 
 template <typename T>
-__device__ __forceinline__ void wind_item(const Solve &S, int pd, int blk) {
+__device__ __forceinline__ void wind_item(const Solve &S, int pd, int blk, int k) {
   const csadv_solve_desc &D = S.d;
-  if ((D.stop > 0 && D.ctl[1] >= D.stop) || D.ctl[0]) return;       // solve finished or halted
-  if (D.nbasis == 1) wind_edges<T, 1>(S, pd & 7, pd >> 3, blk);
-  else if (D.nbasis == 4) wind_edges<T, 4>(S, pd & 7, pd >> 3, blk);
-  else wind_edges<T, 0>(S, pd & 7, pd >> 3, blk);
+  const int steps = D.ctl[1] + k;                                   // steps completed
+  if ((D.stop > 0 && steps >= D.stop) || D.ctl[0]) return;          // solve finished or halted
+  if (D.nbasis == 1) wind_edges<T, 1>(S, pd & 7, pd >> 3, blk, steps);
+  else if (D.nbasis == 4) wind_edges<T, 4>(S, pd & 7, pd >> 3, blk, steps);
+  else wind_edges<T, 0>(S, pd & 7, pd >> 3, blk, steps);
 }
 
 // Workgroup b takes item b of the wind work list (wind_list: the time-dependent solves first, so
@@ -617,15 +671,15 @@ __device__ __forceinline__ void wind_item(const Solve &S, int pd, int blk) {
 template <typename T>
 __global__ __launch_bounds__(BLOCK) void k_wind_avg(const Solve *solves, const int4 *list) {
   const int4 it = list[blockIdx.x];
-  wind_item<T>(solves[it.x], it.y, it.z);
+  wind_item<T>(solves[it.x], it.y, it.z, 0);
 }
 
 // A handle of one solve: the descriptor travels in the kernel arguments; grid (blocks, 12 = panel
-// and direction).
+// and direction); k: steps of the running sequence that the counter does not hold yet.
 template <typename T>
-__global__ __launch_bounds__(BLOCK) void k_wind_avg1(const Solve one) {
+__global__ __launch_bounds__(BLOCK) void k_wind_avg1(const Solve one, int k) {
   const int y = blockIdx.y;
-  wind_item<T>(one, y % 6 + 8 * (y / 6), blockIdx.x);
+  wind_item<T>(one, y % 6 + 8 * (y / 6), blockIdx.x, k);
 }
 
 // ------------------------------------------------------------------ diagnostics
@@ -812,13 +866,15 @@ int ghost_fill(csadv_t *h, hipStream_t st) {
 
 namespace {
 
+// The step kernel; k: its place in the running sequence of steps that fill their own ghosts, or
+// kPlain after the ghost kernel.
 template <typename T>
-hipError_t launch_step_dt(csadv_t *h, hipStream_t st) {
+hipError_t launch_step_dt(csadv_t *h, hipStream_t st, int k, bool keep = false) {
   switch (h->recon) {
-    case 1: return launch_step_r<T, 1>(h, st);
-    case 2: return launch_step_r<T, 2>(h, st);
-    case 4: return launch_step_r<T, 4>(h, st);
-    default: return launch_step_r<T, 3>(h, st);
+    case 1: return launch_step_r<T, 1>(h, st, k, keep);
+    case 2: return launch_step_r<T, 2>(h, st, k, keep);
+    case 4: return launch_step_r<T, 4>(h, st, k, keep);
+    default: return launch_step_r<T, 3>(h, st, k, keep);
   }
 }
 
@@ -848,13 +904,13 @@ int step_ghosts(csadv_t *h, hipStream_t st) {
 }
 
 // The winds of the step: of the time-dependent solves, or of every solve (wind init).
-int wind_avg(csadv_t *h, hipStream_t st, bool all) {
+int wind_avg(csadv_t *h, hipStream_t st, bool all, int k = 0) {
   if (h->desc.size() == 1) {
     const csadv_solve_desc &d = h->desc[0];
     if (!all && (!d.unsteady || own_wind(d))) return CSADV_OK;
     const dim3 grid(wind_blocks(d.N), 12);
-    if (h->dtype == CSADV_F64) hipLaunchKernelGGL(k_wind_avg1<double>, grid, dim3(BLOCK), 0, st, h->host[0]);
-    else hipLaunchKernelGGL(k_wind_avg1<float>, grid, dim3(BLOCK), 0, st, h->host[0]);
+    if (h->dtype == CSADV_F64) hipLaunchKernelGGL(k_wind_avg1<double>, grid, dim3(BLOCK), 0, st, h->host[0], k);
+    else hipLaunchKernelGGL(k_wind_avg1<float>, grid, dim3(BLOCK), 0, st, h->host[0], k);
   } else {
     const int n = all ? h->nwwork : h->nwunsteady;
     if (!n) return CSADV_OK;
@@ -862,6 +918,38 @@ int wind_avg(csadv_t *h, hipStream_t st, bool all) {
     else hipLaunchKernelGGL(k_wind_avg<float>, dim3(n), dim3(BLOCK), 0, st, h->dev, h->wwork);
   }
   HIPCHK(h, hipGetLastError());
+  return CSADV_OK;
+}
+
+// Whether the steps of the handle fill their own ghosts (self_fill), with two buffers for the mass-
+// fixer partials of alternating steps.
+int plan_self(csadv_t *h, hipStream_t st) {
+  h->self = false;
+  if (h->general || h->host.size() != 1 || !self_fill(h->host[0])) return CSADV_OK;
+  const Solve &S = h->host[0];
+  if ((uintptr_t)S.d.lagw % 16 != 0) return CSADV_OK;   // (its weights are read in pairs)
+  const int64_t n = (int64_t)S.part_per_tracer * S.d.ntr;
+  if (n > h->nspart) {
+    if (h->spart) (void)hipFree(h->spart);
+    h->spart = nullptr;
+    h->nspart = 0;
+    HIPCHK(h, hipMalloc(&h->spart, sizeof(double) * (2 * n + 1)));
+    h->nspart = n;
+  }
+  int32_t ok = 1, *flag = reinterpret_cast<int32_t *>(h->spart + 2 * h->nspart);
+  HIPCHK(h, hipMemcpyAsync(flag, &ok, sizeof(ok), hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_check_recipes, dim3(32), dim3(BLOCK), 0, st, S, flag);
+  HIPCHK(h, hipGetLastError());
+  int32_t o[24 * 7];
+  HIPCHK(h, hipMemcpyAsync(&ok, flag, sizeof(ok), hipMemcpyDeviceToHost, st));
+  HIPCHK(h, hipMemcpyAsync(o, S.d.orient, sizeof(o), hipMemcpyDeviceToHost, st));
+  HIPCHK(h, hipStreamSynchronize(st));
+  h->sides.resize(24);
+  for (int t = 0; t < 24; ++t) {
+    const int32_t *r = o + 7 * t;
+    h->sides[t] = {r[0] * (int)S.pstride + r[4] * S.d.ld + r[1], r[5] * S.d.ld + r[2], r[6] * S.d.ld + r[3]};
+  }
+  h->self = ok != 0;
   return CSADV_OK;
 }
 
@@ -876,7 +964,7 @@ int upload_plan(csadv_t *h, hipStream_t st) {
     S.ftx = S.fty = nullptr;
     if (S.mode == kTab) {
       S.ftx = h->ftab[s];
-      S.fty = static_cast<char *>(h->ftab[s]) + flux_x_elems(d.N, d.split) * (d.dtype == CSADV_F64 ? 8 : 4);
+      S.fty = static_cast<char *>(h->ftab[s]) + flux_x_elems(d.N, d.split) * 8;
     }
     h->mode = s == 0 || h->mode == S.mode ? S.mode : (h->rk2 ? kMixed2 : kMixed);
   }
@@ -915,7 +1003,7 @@ int upload_plan(csadv_t *h, hipStream_t st) {
   }
   HIPCHK(h, hipMemcpyAsync(h->dev, h->host.data(), sizeof(Solve) * nsolve, hipMemcpyHostToDevice, st));
   HIPCHK(h, hipStreamSynchronize(st));   // the lists above are host memory of this call
-  return CSADV_OK;
+  return plan_self(h, st);
 }
 
 }  // namespace
@@ -930,9 +1018,7 @@ int csadv_work_bytes(int32_t N, int32_t dtype, int64_t *bytes) { return work_byt
 
 int csadv_tile_rows(int32_t tile) { return tile_rows(tile); }
 
-int csadv_flux_table_bytes(int32_t N, int32_t dtype, int32_t split, int64_t *bytes) {
-  return flux_table_bytes(N, dtype, split, bytes);
-}
+int csadv_flux_table_bytes(int32_t N, int32_t split, int64_t *bytes) { return flux_table_bytes(N, split, bytes); }
 
 int csadv_create(const csadv_solve_desc *solves, int32_t nsolve, int32_t tile, csadv_t **out) {
   if (!out) return CSADV_E_ARG;
@@ -1034,6 +1120,7 @@ int csadv_bind_flux_tables(csadv_t *h, void *const *tables, void *stream) {
   for (int s = 0; s < ns; ++s) {
     if (!tables || !tables[s]) continue;
     const csadv_solve_desc &d = h->desc[s];
+    if (d.dtype != CSADV_F64) return fail(h, CSADV_E_ARG, "flux tables belong to FP64 solves");
     if ((uintptr_t)tables[s] % 16 != 0) return fail(h, CSADV_E_ARG, "flux tables must be 16-byte aligned");
     if (d.ld != general_ld(d.N) || d.ldu != general_ldu(d.N))
       return fail(h, CSADV_E_ARG, "flux tables expect ld = round_up(N+8, 4) and ldu = round_up(N+9, 4)");
@@ -1168,26 +1255,38 @@ int diagnostics(csadv_t *h, int solve, int tracer0, int ntracers, const double *
   return CSADV_OK;
 }
 
+// Whether a sequence of n steps fills its own ghosts: one step alone takes the ghost kernel instead
+// of the one that ends a sequence.
+bool self_steps(const csadv_t *h, int n) { return h->self && n > 1; }
+
 // The kernels of one step, in order, on stream st (event pairs only when armed).
-int enqueue_step(csadv_t *h, hipStream_t st, bool allow_prof) {
+// Step k of the n that csadv_step or a graph enqueues one after another (end_steps ends them).
+int enqueue_step(csadv_t *h, hipStream_t st, bool allow_prof, int k, int n) {
+  const bool self = self_steps(h, n);
   if (h->general) {
     const int rc = wind_avg(h, st, false);
     if (rc) return rc;
     return h->dtype == CSADV_F64 ? enqueue_general_t<double>(h, st) : enqueue_general_t<float>(h, st);
   }
-  int rc = wind_avg(h, st, false);
+  int rc = wind_avg(h, st, false, self ? k : 0);
   if (rc) return rc;
-  rc = step_ghosts(h, st);
+  if (!self) rc = step_ghosts(h, st);
   if (rc) return rc;
   const bool prof = allow_prof && 2 * (h->ev_used + 1) <= (int)h->ev.size();
   if (prof) HIPCHK(h, hipEventRecord(h->ev[2 * h->ev_used], st));
-  hipError_t e = h->dtype == CSADV_F64 ? launch_step_dt<double>(h, st) : launch_step_dt<float>(h, st);
+  hipError_t e = h->dtype == CSADV_F64 ? launch_step_dt<double>(h, st, self ? k : kPlain, k >= n - 2)
+                                          : launch_step_dt<float>(h, st, self ? k : kPlain, k >= n - 2);
   if (e != hipSuccess) return fail(h, CSADV_E_HIP, std::string("step kernel: ") + hipGetErrorString(e));
   if (prof) {
     HIPCHK(h, hipEventRecord(h->ev[2 * h->ev_used + 1], st));
     ++h->ev_used;
   }
-  if (h->mfaf) {   // MF-AF: the cube-edge flux averages into the boundary cells
+  if (h->mfaf && self) {
+    const dim3 grid((6 * 4 * (h->desc[0].N - 1) + BLOCK - 1) / BLOCK, h->desc[0].ntr);
+    if (h->dtype == CSADV_F64) hipLaunchKernelGGL(k_af_fix1<double>, grid, dim3(BLOCK), 0, st, h->host[0], k);
+    else hipLaunchKernelGGL(k_af_fix1<float>, grid, dim3(BLOCK), 0, st, h->host[0], k);
+    HIPCHK(h, hipGetLastError());
+  } else if (h->mfaf) {   // MF-AF: the cube-edge flux averages into the boundary cells
     int maxN = 0, maxtr = 1;
     for (auto &d : h->desc) { maxN = std::max(maxN, d.N); maxtr = std::max(maxtr, d.ntr); }
     const dim3 grid((6 * 4 * (maxN - 1) + BLOCK - 1) / BLOCK, (int)h->desc.size(), maxtr);
@@ -1198,12 +1297,21 @@ int enqueue_step(csadv_t *h, hipStream_t st, bool allow_prof) {
   return CSADV_OK;
 }
 
+// End of a sequence of n enqueued steps.
+int end_steps(csadv_t *h, hipStream_t st, int n) {
+  if (!self_steps(h, n)) return CSADV_OK;
+  hipLaunchKernelGGL(k_advance, dim3(1), dim3(BLOCK), 0, st, h->host[0], n, h->spart, h->spart + h->nspart);
+  HIPCHK(h, hipGetLastError());
+  return CSADV_OK;
+}
+
 // Capture graph_steps steps on the private stream and instantiate them.
 int build_graph(csadv_t *h) {
   if (!h->cap) HIPCHK(h, hipStreamCreateWithFlags(&h->cap, hipStreamNonBlocking));
   HIPCHK(h, hipStreamBeginCapture(h->cap, hipStreamCaptureModeRelaxed));
   int rc = CSADV_OK;
-  for (int k = 0; k < h->graph_steps && rc == CSADV_OK; ++k) rc = enqueue_step(h, h->cap, false);
+  for (int k = 0; k < h->graph_steps && rc == CSADV_OK; ++k) rc = enqueue_step(h, h->cap, false, k, h->graph_steps);
+  if (rc == CSADV_OK) rc = end_steps(h, h->cap, h->graph_steps);
   hipGraph_t g = nullptr;
   hipError_t e = hipStreamEndCapture(h->cap, &g);
   if (rc != CSADV_OK) {
@@ -1247,10 +1355,13 @@ int csadv_step(csadv_t *h, int32_t nsteps, void *stream) {
       HIPCHK(h, hipGraphLaunch(h->gexec, st));
     }
   }
+  const int k0 = k;
   for (; k < nsteps; ++k) {
-    const int rc = enqueue_step(h, st, true);
+    const int rc = enqueue_step(h, st, true, k - k0, nsteps - k0);
     if (rc) return rc;
   }
+  const int rc = end_steps(h, st, nsteps - k0);
+  if (rc) return rc;
   for (int s = 0; s < ns; ++s) {
     const int stop = h->desc[s].stop;
     h->done[s] += nsteps;
@@ -1402,7 +1513,7 @@ int csadv_time_step_kernel(csadv_t *h, int32_t reps, void *stream, double *us_pe
   HIPCHK(h, hipStreamBeginCapture(h->cap, hipStreamCaptureModeRelaxed));
   hipError_t e = hipSuccess;
   for (int k = 0; k < reps && e == hipSuccess; ++k)
-    e = h->dtype == CSADV_F64 ? launch_step_dt<double>(h, h->cap) : launch_step_dt<float>(h, h->cap);
+    e = h->dtype == CSADV_F64 ? launch_step_dt<double>(h, h->cap, kRepeat) : launch_step_dt<float>(h, h->cap, kRepeat);
   hipGraph_t g = nullptr;
   const hipError_t ec = hipStreamEndCapture(h->cap, &g);
   if (e != hipSuccess || ec != hipSuccess) {
@@ -1447,8 +1558,8 @@ int csadv_time_step_kernel_rotating(csadv_t *const *handles, int32_t nhandles, i
   hipError_t e = hipSuccess;
   for (int r = 0; r < reps && e == hipSuccess; ++r)
     for (int k = 0; k < nhandles && e == hipSuccess; ++k)
-      e = handles[k]->dtype == CSADV_F64 ? launch_step_dt<double>(handles[k], h0->cap)
-                                         : launch_step_dt<float>(handles[k], h0->cap);
+      e = handles[k]->dtype == CSADV_F64 ? launch_step_dt<double>(handles[k], h0->cap, kRepeat)
+                                         : launch_step_dt<float>(handles[k], h0->cap, kRepeat);
   hipGraph_t g = nullptr;
   const hipError_t ec = hipStreamEndCapture(h0->cap, &g);
   if (e != hipSuccess || ec != hipSuccess) {
@@ -1482,6 +1593,7 @@ void csadv_destroy(csadv_t *h) {
   if (h->work) (void)hipFree(h->work);
   if (h->gwork) (void)hipFree(h->gwork);
   if (h->wwork) (void)hipFree(h->wwork);
+  if (h->spart) (void)hipFree(h->spart);
   if (h->qsets) (void)hipFree(h->qsets);
   if (h->wsets) (void)hipFree(h->wsets);
   if (h->red) (void)hipFree(h->red);

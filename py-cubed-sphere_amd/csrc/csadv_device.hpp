@@ -55,9 +55,56 @@ template <typename T> __device__ __forceinline__ T sgn(T x) { return (x > T(0)) 
 
 // PPM edge values (q_L, q_R) of one cell from its 5-cell window; src/reconstruction_1d.py:26-193.
 //   RECON 1 PPM-0 (CW84 eq. 1.9), 2 PPM-CW84 (monotone), 3 PPM-PL07 (eqs. 41-42), 4 PPM-L04 (B1-B4)
+// The limited schemes (2: limited slopes at c-1, c, c+1, CW84 eqs. 1.7-1.8, a local extremum
+// flattened, eq. 1.10, and overshoots cut; 4: monotone slopes, L04 eq. B1, edges by B3 and B4) as
+// one text for two functions: limited_edges, whose multiply-adds the compiler fuses where it
+// likes, and limited_edges_on, which fuses them within one source expression only, so that its bits do
+// not depend on the kernel around it.
+#define CSADV_LIMITED_EDGES(NAME, CONTRACT) \
+template <typename T, int RECON> \
+__device__ __forceinline__ void NAME(T m2, T m1, T c0, T p1, T p2, T &qL, T &qR) { \
+  CONTRACT \
+  if constexpr (RECON == 2) { \
+ \
+    auto slope = [](T a, T b, T c) { \
+      T d0 = T(0.5) * (c - a), d1 = T(2.0) * (c - b), d2 = T(2.0) * (b - a); \
+      T d = fmin(fabs(d0), fabs(d1)); \
+      d = fmin(d, fabs(d2)) * sgn(d0); \
+      return ((c - b) * (b - a) > T(0)) ? d : T(0); \
+    }; \
+    T sm = slope(m2, m1, c0), s0 = slope(m1, c0, p1), sp = slope(c0, p1, p2); \
+    T R = T(0.5) * (p1 + c0) - (sp - s0) / T(6.0); \
+    T L = T(0.5) * (c0 + m1) - (s0 - sm) / T(6.0); \
+    T dq = R - L, q6 = T(6) * c0 - T(3) * (R + L); \
+    if ((R - c0) * (c0 - L) <= T(0)) { R = c0; L = c0; } \
+    bool over = fabs(dq) < fabs(q6); \
+    T dd = R - L, mm = c0 - T(0.5) * (R + L); \
+    bool left = dd * mm > (dd * dd) / T(6.0); \
+    bool right = -(dd * dd) / T(6.0) > dd * mm; \
+    if (over && left) L = T(3.0) * c0 - T(2.0) * R; \
+    if (over && right) R = T(3.0) * c0 - T(2.0) * L; \
+    qL = L; qR = R; \
+  } else { \
+ \
+    auto mono = [](T a, T b, T c) { \
+      T d = T(0.25) * (c - a); \
+      T mx = fmax(fmax(a, b), c), mn = fmin(fmin(a, b), c); \
+      return fmin(fmin(fabs(d), mx - b), b - mn) * sgn(d); \
+    }; \
+    T dm = mono(m2, m1, c0), d0 = mono(m1, c0, p1), dp = mono(c0, p1, p2); \
+    T R = T(0.5) * (p1 + c0) - (dp - d0) / T(3.0); \
+    T L = T(0.5) * (c0 + m1) - (d0 - dm) / T(3.0); \
+    T s = sgn(T(2.0) * d0); \
+    qL = c0 - fmin(T(2.0) * fabs(d0), fabs(L - c0)) * s; \
+    qR = c0 + fmin(T(2.0) * fabs(d0), fabs(R - c0)) * s; \
+  } \
+}
+CSADV_LIMITED_EDGES(limited_edges, )
+CSADV_LIMITED_EDGES(limited_edges_on, _Pragma("clang fp contract(on)"))
+#undef CSADV_LIMITED_EDGES
+
 template <typename T, int RECON>
 __device__ __forceinline__ void recon_edges(T m2, T m1, T c0, T p1, T p2, T &qL, T &qR) {
-#pragma clang fp contract(on)
   if constexpr (RECON == 3) {
     const T a1 = T(2.0 / 60.0), a2 = T(-13.0 / 60.0), a3 = T(47.0 / 60.0), a4 = T(27.0 / 60.0), a5 = T(-3.0 / 60.0);
     qR = a1 * m2 + a2 * m1 + a3 * c0 + a4 * p1 + a5 * p2;
@@ -66,39 +113,8 @@ __device__ __forceinline__ void recon_edges(T m2, T m1, T c0, T p1, T p2, T &qL,
     const T s7 = T(7.0 / 12.0);
     qR = s7 * (p1 + c0) - (p2 + m1) / T(12.0);
     qL = s7 * (c0 + m1) - (p1 + m2) / T(12.0);
-  } else if constexpr (RECON == 2) {
-    // limited slopes at c-1, c, c+1 (CW84 eqs. 1.7-1.8)
-    auto slope = [](T a, T b, T c) {
-      T d0 = T(0.5) * (c - a), d1 = T(2.0) * (c - b), d2 = T(2.0) * (b - a);
-      T d = fmin(fabs(d0), fabs(d1));
-      d = fmin(d, fabs(d2)) * sgn(d0);
-      return ((c - b) * (b - a) > T(0)) ? d : T(0);
-    };
-    T sm = slope(m2, m1, c0), s0 = slope(m1, c0, p1), sp = slope(c0, p1, p2);
-    T R = T(0.5) * (p1 + c0) - (sp - s0) / T(6.0);
-    T L = T(0.5) * (c0 + m1) - (s0 - sm) / T(6.0);
-    T dq = R - L, q6 = T(6) * c0 - T(3) * (R + L);
-    if ((R - c0) * (c0 - L) <= T(0)) { R = c0; L = c0; }     // local extremum: flatten (eq. 1.10)
-    bool over = fabs(dq) < fabs(q6);
-    T dd = R - L, mm = c0 - T(0.5) * (R + L);
-    bool left = dd * mm > (dd * dd) / T(6.0);
-    bool right = -(dd * dd) / T(6.0) > dd * mm;
-    if (over && left) L = T(3.0) * c0 - T(2.0) * R;
-    if (over && right) R = T(3.0) * c0 - T(2.0) * L;
-    qL = L; qR = R;
   } else {
-    // monotone slope (L04 eq. B1) at c-1, c, c+1
-    auto mono = [](T a, T b, T c) {
-      T d = T(0.25) * (c - a);
-      T mx = fmax(fmax(a, b), c), mn = fmin(fmin(a, b), c);
-      return fmin(fmin(fabs(d), mx - b), b - mn) * sgn(d);
-    };
-    T dm = mono(m2, m1, c0), d0 = mono(m1, c0, p1), dp = mono(c0, p1, p2);
-    T R = T(0.5) * (p1 + c0) - (dp - d0) / T(3.0);
-    T L = T(0.5) * (c0 + m1) - (d0 - dm) / T(3.0);
-    T s = sgn(T(2.0) * d0);
-    qL = c0 - fmin(T(2.0) * fabs(d0), fabs(L - c0)) * s;   // eq. B3
-    qR = c0 + fmin(T(2.0) * fabs(d0), fabs(R - c0)) * s;   // eq. B4
+    limited_edges<T, RECON>(m2, m1, c0, p1, p2, qL, qR);
   }
 }
 
@@ -179,7 +195,7 @@ __device__ __forceinline__ Cell<T> cell_of(T m2, T m1, T c0, T p1, T p2) {
     c.a = __builtin_elementwise_fma(T(L::r), p2 + m2, p1 + m1);
     c.b = __builtin_elementwise_fma(T(L::t), p2 - m2, p1 - m1);
   } else {
-    recon_edges<T, RECON>(m2, m1, c0, p1, p2, c.a, c.b);
+    limited_edges_on<T, RECON>(m2, m1, c0, p1, p2, c.a, c.b);
   }
   return c;
 }
@@ -200,11 +216,9 @@ template <typename T>
 struct FluxEntry {
   T w0, w1, w2, h;
 };
-__device__ __forceinline__ float tag_low(float v, bool b) { return __uint_as_float((__float_as_uint(v) & ~1u) | (b ? 1u : 0u)); }
 __device__ __forceinline__ double tag_low(double v, bool b) {
   return __longlong_as_double((__double_as_longlong(v) & ~1ll) | (b ? 1ll : 0ll));
 }
-__device__ __forceinline__ bool low_tag(float v) { return __float_as_uint(v) & 1u; }
 __device__ __forceinline__ bool low_tag(double v) { return (unsigned)__double_as_longlong(v) & 1u; }
 
 // The weights of an edge with Courant number c (s as above), gA / gD the edge metrics at the edge
@@ -245,7 +259,7 @@ __device__ __forceinline__ EdgeW<T> edge_weights(bool up, T c, T s, T gA, T gD, 
       w.w2 = -cg * (s * om);
     }
   }
-  if constexpr (!std::is_same<T, float>::value) w.w2 = tag_low(w.w2, up);   // (as a table holds it)
+  w.w2 = tag_low(w.w2, up);   // (as a table holds it)
   return w;
 }
 
@@ -367,18 +381,6 @@ __device__ __forceinline__ void st_buf(__amdgpu_buffer_rsrc_t r, uint32_t byte_o
 
 // Entry at byte offset off of a flux table (buffer loads: three words at once need no alignment
 // padding; the buffer covers one panel's table, under 2^32 bytes).
-typedef unsigned int csadv_u32x3 __attribute__((ext_vector_type(3)));
-typedef unsigned int csadv_u32x4 __attribute__((ext_vector_type(4)));
-template <int NW>
-__device__ __forceinline__ FluxEntry<float> ld_flux(__amdgpu_buffer_rsrc_t r, uint32_t off, float) {
-  if constexpr (NW == 3) {
-    const csadv_u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
-    return {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), 0.f};
-  } else {
-    const csadv_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
-    return {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
-  }
-}
 template <int NW>
 __device__ __forceinline__ FluxEntry<double> ld_flux(__amdgpu_buffer_rsrc_t r, uint32_t off, double) {
   typedef double f64x2 __attribute__((ext_vector_type(2)));
@@ -486,9 +488,56 @@ __device__ __forceinline__ int touch_solve(const Solve &S, int v) {
   return v;
 }
 
+// Sum over a wavefront, complete in lane 0, in the order of shuffles down by 32, 16, 8, 4, 2, 1:
+// the halves and the rows of 16 by gfx950's lane swaps, within a row by DPP shifts (a tenth of the
+// latency of shuffles through the LDS crossbar, on the critical path at both ends of a march).
+__device__ __forceinline__ double lane_up32(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  const unsigned l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false)[1];
+  const unsigned h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false)[1];
+  return __longlong_as_double(((long long)h << 32) | l);
+}
+__device__ __forceinline__ double lane_up16(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  const unsigned l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false)[1];
+  const unsigned h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false)[1];
+  return __longlong_as_double(((long long)h << 32) | l);
+}
 __device__ __forceinline__ double warp_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  v += lane_up32(v);
+  v += lane_up16(v);
+  v += dpp_move<0x108>(v);   // row_shl:8 -- lane i takes lane i + 8 of its row
+  v += dpp_move<0x104>(v);
+  v += dpp_move<0x102>(v);
+  v += dpp_move<0x101>(v);
   return v;
 }
+// The same, in every lane.
+__device__ __forceinline__ double wave_total(double v) {
+  const long long b = __double_as_longlong(warp_sum(v));
+  const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Mass-fixer correction total C after `steps` steps, from the stored totals c0 / c1 (slots of
+// even / odd steps) and the partials' sum: with the partials of the last step pending,
+// C = C(steps - 1) + dt m0 / a2, m0 = sum of div g over the interior
+// (src/discrete_operators.py:98-101); otherwise C is the stored total of this step.
+__device__ __forceinline__ double corr_total(double dt, double a2, double c0, double c1, double sum, int pending,
+                                             int steps) {
+  const double held = (steps & 1) ? c1 : c0, prev = (steps & 1) ? c0 : c1;
+  return pending ? prev + dt * sum / a2 : held;
+}
+
+// A strip ghost's value: its four sources in recipe order, every product fused.
+__device__ __forceinline__ double strip_sum(double v0, double v1, double v2, double v3, double w0, double w1, double w2,
+                                            double w3) {
+  return fma(v3, w3, fma(v2, w2, fma(v1, w1, v0 * w0)));
+}
+
+// Row m (0 .. 5) of the corner ghosts outside a panel: the three below it, the three above.
+__device__ __forceinline__ int corner_row(int m, int N) { return m < 3 ? NG - 3 + m : N + NG + m - 3; }
 
 }  // namespace csadv

@@ -34,6 +34,10 @@ struct csadv_s {
   bool general = false;           // ET-S72 / ET-PL07: the general step
   bool mfaf = false;              // a fused-step solve with MF-AF: k_af_fix after the step kernel
   int mode = kRk1;                // FluxMode of every solve, or kMixed
+  bool self = false;              // one solve whose step kernel fills its own ghosts (self_fill)
+  double *spart = nullptr;        // self: the mass-fixer partials of alternating steps, 2 x nspart
+  int64_t nspart = 0;
+  std::vector<SelfSide> sides;    // self: the ghost sources of the 24 panel sides
   std::vector<void *> ftab;       // the bound flux tables, one per solve (null: none)
   double *red = nullptr;          // diagnostics scratch: partials and outputs (diag_scratch_words)
   int red_tracers = 1;            // tracers the diagnostics scratch holds (the largest ntr)
@@ -68,9 +72,12 @@ inline int64_t diag_scratch_words(int ntracers) {
 // Full 4-layer duo-grid ghost fill of every tracer's current buffer (csadv.hip).
 int ghost_fill(csadv_t *h, hipStream_t st);
 
-// The fused step kernel of every solve for reconstruction R (step_<dtype>_r<R>.hip).
+// The fused step kernel of every solve for reconstruction R (step_<dtype>_r<R>.hip); k: its place in
+// a sequence of steps that fill their own ghosts, kPlain after the ghost kernel, kRepeat the last
+// step once more; keep: such a step stores its ghosts, too.
+constexpr int kPlain = -2, kRepeat = -1;
 template <typename T, int R>
-hipError_t launch_step_r(csadv_t *h, hipStream_t st);
+hipError_t launch_step_r(csadv_t *h, hipStream_t st, int k, bool keep);
 
 // One general step of every solve with splitting SP (general_<dtype>_s<SP>.hip), and by the
 // handle's splitting.

@@ -165,9 +165,9 @@ int work_bytes(int N, int dtype, int64_t *bytes) {
   return CSADV_OK;
 }
 
-int flux_table_bytes(int N, int dtype, int split, int64_t *bytes) {
-  if (!bytes || N < 8 || N > 8192 || (dtype != CSADV_F64 && dtype != CSADV_F32) || split < 1 || split > 3) return CSADV_E_ARG;
-  *bytes = flux_elems(N, split) * (dtype == CSADV_F64 ? 8 : 4);
+int flux_table_bytes(int N, int split, int64_t *bytes) {
+  if (!bytes || N < 8 || N > 8192 || split < 1 || split > 3) return CSADV_E_ARG;
+  *bytes = flux_elems(N, split) * 8;
   return CSADV_OK;
 }
 

@@ -37,8 +37,8 @@ constexpr int kNumTiles = sizeof(kSegRows) / sizeof(kSegRows[0]);
 //   kWind       formed in the step kernel from a one-field time-dependent wind (RK1): the FP64
 //               basis times its coefficient at the step's time (own_wind)
 //   kRk1, kRk2  formed in the step kernel from the wind arrays
-// kMixed, kMixed2: a handle of RK1 (RK2) solves that differ, each by its own mode.  In FP64 all give
-// the same bits; in FP32 a table's weights are formed in FP64 and rounded once.
+// kMixed, kMixed2: a handle of RK1 (RK2) solves that differ, each by its own mode.  All give the
+// same bits.
 enum FluxMode : int { kRk1 = 0, kRk2 = 1, kWind = 2, kTab = 3, kMixed = 4, kMixed2 = 5 };
 
 // Device copy of one solve: the public descriptor plus derived strides.
@@ -125,7 +125,21 @@ inline bool own_wind(const csadv_solve_desc &d) {
   return !is_general(d) && d.unsteady && d.dp == 1 && d.nbasis == 1;
 }
 
-// Flux tables: per edge the weights of its upwind flux (EdgeW, csadv_device.hpp) and, with the
+// Whether consecutive steps of a handle of this one solve fill their own ghosts in the step kernel,
+// with no ghost kernel between them (csadv_step.hpp): a small solve's step is bound by its launches
+// and chains of loads.  With at most one wavefront per SIMD (1024) it pays: N = 24 .. 192 FP64 5-10%
+// of a step, 384 (1008 wavefronts) 6%, without the mass fixer's sum 12-18%.  With more the ghost
+// stage's registers leave too few resident (three FP32 tracers at N = 384, 3024 wavefronts: 19.8 us
+// -> 27.8), and over long segments the march's reads of the ghosts cost more than the ghost kernel
+// (N = 256, 32 rows: 17.7 -> 18.7 us).
+constexpr int kSelfMaxWaves = 1024, kSelfMaxRows = 16;
+inline bool self_fill(const Solve &S) {
+  return !is_general(S.d) && S.part_per_tracer * S.d.ntr <= kSelfMaxWaves && S.seg_l <= kSelfMaxRows;
+}
+struct SelfSide {
+  int32_t base, ds, rs;              // element of a (panel, side)'s source at depth d, row r: base + d ds + r rs
+};
+// Flux tables (FP64 solves): per edge the weights of its upwind flux (EdgeW, csadv_device.hpp) and, with the
 // splittings that need it, the metric-weighted Courant number: [6][M][ldu][flux_words] at the
 // x-edges, then [6][M + 1][ld][flux_words] at the y-edges.
 CSADV_HD constexpr int flux_words(int split) { return split == 1 ? 3 : 4; }
@@ -182,6 +196,6 @@ std::vector<Item> wind_list(const std::vector<Solve> &solves, int &unsteady);
 int partials_per_tracer(int N, int tile);
 int work_bytes(int N, int dtype, int64_t *bytes);
 int tile_rows(int tile);
-int flux_table_bytes(int N, int dtype, int split, int64_t *bytes);
+int flux_table_bytes(int N, int split, int64_t *bytes);
 
 }  // namespace csadv

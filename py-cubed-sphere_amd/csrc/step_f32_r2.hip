@@ -2,4 +2,4 @@
 // reconstruction, so that the library's kernels compile in parallel).
 #include "csadv_step.hpp"
 
-template hipError_t launch_step_r<float, 2>(csadv_t *h, hipStream_t st);
+template hipError_t launch_step_r<float, 2>(csadv_t *h, hipStream_t st, int k, bool keep);

@@ -70,7 +70,7 @@ def load():
     lib.csadv_work_bytes.argtypes = [i32, i32, ctypes.POINTER(ctypes.c_int64)]
     lib.csadv_update.argtypes = [vp, ctypes.POINTER(SolveDesc), i32, vp]
     lib.csadv_wind_init.argtypes = [vp, vp]
-    lib.csadv_flux_table_bytes.argtypes = [i32, i32, i32, ctypes.POINTER(ctypes.c_int64)]
+    lib.csadv_flux_table_bytes.argtypes = [i32, i32, ctypes.POINTER(ctypes.c_int64)]
     lib.csadv_bind_flux_tables.argtypes = [vp, ctypes.POINTER(vp), vp]
     lib.csadv_refresh_winds.argtypes = [vp, vp]
     lib.csadv_ghost_fill.argtypes = [vp, vp]

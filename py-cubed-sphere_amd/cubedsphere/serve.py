@@ -137,7 +137,7 @@ class Server:
         cells = 6 * M * ld
         b = 2 * ntr * cells * s + 6 * M * ldu * s + 6 * (M + 1) * ld * s          # state, winds
         b += K * (6 * M * ldu + 6 * (M + 1) * ld) * 8 + K * 2 * cells * 8       # basis, scratch
-        if req.case.steady:                       # flux table (none for a large FP64 solve: an upper bound)
+        if req.case.steady and req.dtype == "f64":       # flux table (none for a large solve: an upper bound)
             b += (6 * M * ldu + 6 * (M + 1) * ld) * 3 * s
         b += req.nsteps * 2 * K * 8 + ntr * 6 * req.N * req.N // 16 * 8          # coefficients, partials
         return b

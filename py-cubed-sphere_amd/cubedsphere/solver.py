@@ -128,19 +128,17 @@ def time_step_kernel_rotating(solves, reps=20):
     return us.value
 
 
-# An FP64 table read from beyond the 32 MB of L2 costs more than forming its weights: steps with and
-# without it took 14.2 / 15.2 us at N = 256 (19 MB), 15.4 / 16.6 at 320 (30 MB), 17.5 / 17.3 at 384
-# (42 MB) and 25.5 / 22.7 at 512.  In FP32 the weights cost as many instructions for half the bytes:
-# 26.8 / 26.9 us at N = 768 with one tracer (85 MB), 57.7 / 67.5 with four.
-FLUX_TABLE_MAX_F64 = 36 << 20
+# A table read from beyond the 32 MB of L2 costs more than forming its weights: steps with and without
+# it took 14.2 / 15.2 us at N = 256 (19 MB), 15.4 / 16.6 at 320 (30 MB), 17.5 / 17.3 at 384 (42 MB)
+# and 25.5 / 22.7 at 512.
+FLUX_TABLE_MAX = 36 << 20
 
 
-def flux_table_bytes(N, dtype, split):
-    """Bytes of a steady fused-step solve's flux table, 0 where the step forms the weights."""
+def flux_table_bytes(N, split):
+    """Bytes of a steady FP64 fused-step solve's flux table, 0 where the step forms the weights."""
     n = ctypes.c_int64()
-    _lib.check(_lib.load().csadv_flux_table_bytes(N, _lib.CSADV_F64 if dtype == "f64" else _lib.CSADV_F32, split,
-                                                  ctypes.byref(n)), None, "csadv_flux_table_bytes")
-    return 0 if dtype == "f64" and n.value > FLUX_TABLE_MAX_F64 else int(n.value)
+    _lib.check(_lib.load().csadv_flux_table_bytes(N, split, ctypes.byref(n)), None, "csadv_flux_table_bytes")
+    return int(n.value) if n.value <= FLUX_TABLE_MAX else 0
 
 
 _TABLES = {}
@@ -267,18 +265,19 @@ class Advection:
             _lib.check(code, None, "csadv_work_bytes")
             self.work = torch.zeros(int(nbytes.value), device=dev, dtype=torch.uint8)
         # a steady solve's flux weights, kept in a table where that beats forming them in every step
-        nbytes = flux_table_bytes(N, self.dtype, self.opts["split"]) if self.case.steady and not general else 0
+        use = self.case.steady and self.dtype == "f64" and not general
+        nbytes = flux_table_bytes(N, self.opts["split"]) if use else 0
         self.flux_table = torch.zeros(nbytes, device=dev, dtype=torch.uint8) if nbytes else None
         if not general and self.opts["mf"] == 2:
             self.work = torch.zeros(ntr * 24 * N, device=dev, dtype=td)
 
     @staticmethod
     def bind_flux_tables(lib, handle, members, stream, fill=False):
-        """Hand the members' flux tables to their handle (csadv_bind_flux_tables).  FP64 members
-        step with them only where all of them together stay in cache (their weights formed in the
-        step have the same bits); ``fill``: bound to be filled by csadv_wind_init."""
+        """Hand the members' flux tables to their handle (csadv_bind_flux_tables).  The members step
+        with them only where all of them together stay in cache (weights formed in the step have the
+        same bits); ``fill``: bound to be filled by csadv_wind_init."""
         total = sum(m.flux_table.numel() for m in members if m.flux_table is not None)
-        if total == 0 or (members[0].dtype == "f64" and total > FLUX_TABLE_MAX_F64 and not fill):
+        if total == 0 or (total > FLUX_TABLE_MAX and not fill):
             return
         tabs = (ctypes.c_void_p * len(members))(*[m.flux_table.data_ptr() if m.flux_table is not None else None
                                                   for m in members])
