@@ -53,6 +53,23 @@ __device__ __forceinline__ void ghost_target(int side, int d, int k, int N, int 
 
 template <typename T> __device__ __forceinline__ T sgn(T x) { return (x > T(0)) ? T(1) : ((x < T(0)) ? T(-1) : T(0)); }
 
+// x / B for a small constant B, with the division's own rounding in three operations (a division
+// takes about ten): q is x times the rounded reciprocal, and one fma with the exact remainder
+// x - B q corrects it (Markstein's theorem; checked against the division for every FP32 mantissa
+// and 2e8 FP64 ones for B = 3, 6, 12).
+template <int B, typename T>
+__device__ __forceinline__ T div_const(T x) {
+  const T y = T(1.0 / B), q = x * y;
+  return __builtin_elementwise_fma(__builtin_elementwise_fma(T(-B), q, x), y, q);
+}
+
+// 1 / x, x near 1 (FP64): the hardware's estimate (24 bits) and two Newton steps, within an ulp.
+__device__ __forceinline__ double recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+
 // PPM edge values (q_L, q_R) of one cell from its 5-cell window; src/reconstruction_1d.py:26-193.
 //   RECON 1 PPM-0 (CW84 eq. 1.9), 2 PPM-CW84 (monotone), 3 PPM-PL07 (eqs. 41-42), 4 PPM-L04 (B1-B4)
 // The limited schemes (2: limited slopes at c-1, c, c+1, CW84 eqs. 1.7-1.8, a local extremum
@@ -73,14 +90,15 @@ __device__ __forceinline__ void NAME(T m2, T m1, T c0, T p1, T p2, T &qL, T &qR)
       return ((c - b) * (b - a) > T(0)) ? d : T(0); \
     }; \
     T sm = slope(m2, m1, c0), s0 = slope(m1, c0, p1), sp = slope(c0, p1, p2); \
-    T R = T(0.5) * (p1 + c0) - (sp - s0) / T(6.0); \
-    T L = T(0.5) * (c0 + m1) - (s0 - sm) / T(6.0); \
+    T R = T(0.5) * (p1 + c0) - div_const<6>(sp - s0); \
+    T L = T(0.5) * (c0 + m1) - div_const<6>(s0 - sm); \
     T dq = R - L, q6 = T(6) * c0 - T(3) * (R + L); \
     if ((R - c0) * (c0 - L) <= T(0)) { R = c0; L = c0; } \
     bool over = fabs(dq) < fabs(q6); \
     T dd = R - L, mm = c0 - T(0.5) * (R + L); \
-    bool left = dd * mm > (dd * dd) / T(6.0); \
-    bool right = -(dd * dd) / T(6.0) > dd * mm; \
+    const T d6 = div_const<6>(dd * dd); \
+    bool left = dd * mm > d6; \
+    bool right = -d6 > dd * mm; \
     if (over && left) L = T(3.0) * c0 - T(2.0) * R; \
     if (over && right) R = T(3.0) * c0 - T(2.0) * L; \
     qL = L; qR = R; \
@@ -92,8 +110,8 @@ __device__ __forceinline__ void NAME(T m2, T m1, T c0, T p1, T p2, T &qL, T &qR)
       return fmin(fmin(fabs(d), mx - b), b - mn) * sgn(d); \
     }; \
     T dm = mono(m2, m1, c0), d0 = mono(m1, c0, p1), dp = mono(c0, p1, p2); \
-    T R = T(0.5) * (p1 + c0) - (dp - d0) / T(3.0); \
-    T L = T(0.5) * (c0 + m1) - (d0 - dm) / T(3.0); \
+    T R = T(0.5) * (p1 + c0) - div_const<3>(dp - d0); \
+    T L = T(0.5) * (c0 + m1) - div_const<3>(d0 - dm); \
     T s = sgn(T(2.0) * d0); \
     qL = c0 - fmin(T(2.0) * fabs(d0), fabs(L - c0)) * s; \
     qR = c0 + fmin(T(2.0) * fabs(d0), fabs(R - c0)) * s; \
@@ -111,8 +129,8 @@ __device__ __forceinline__ void recon_edges(T m2, T m1, T c0, T p1, T p2, T &qL,
     qL = a5 * m2 + a4 * m1 + a3 * c0 + a2 * p1 + a1 * p2;
   } else if constexpr (RECON == 1) {
     const T s7 = T(7.0 / 12.0);
-    qR = s7 * (p1 + c0) - (p2 + m1) / T(12.0);
-    qL = s7 * (c0 + m1) - (p1 + m2) / T(12.0);
+    qR = s7 * (p1 + c0) - div_const<12>(p2 + m1);
+    qL = s7 * (c0 + m1) - div_const<12>(p1 + m2);
   } else {
     limited_edges<T, RECON>(m2, m1, c0, p1, p2, qL, qR);
   }
@@ -405,7 +423,8 @@ template <typename T>
 __device__ __forceinline__ T split_update(int split, T Q, T dF, T g, T rg, T c1, T c2) {
   if (split == 1) return (Q * g + T(0.5) * dF) * rg;
   if (split == 2) return (Q * g + T(0.5) * dF + T(0.5) * (c1 - c2) * Q) * rg;
-  return T(0.5) * (Q + (Q + dF) / (T(1.0) - (c1 - c2)));
+  if constexpr (!std::is_same<T, float>::value) return T(0.5) * (Q + (Q + dF) * recip(T(1.0) - (c1 - c2)));
+  else return T(0.5) * (Q + (Q + dF) / (T(1.0) - (c1 - c2)));
 }
 
 // The split's half-step of one cell (src/discrete_operators.py:49-73) in two parts: a factor that
@@ -415,7 +434,7 @@ __device__ __forceinline__ T split_update(int split, T Q, T dF, T g, T rg, T c1,
 template <typename T, int SPLIT>
 __device__ __forceinline__ T half_factor(T rg, T dc) {
 #pragma clang fp contract(off)
-  if constexpr (SPLIT == 3) return T(0.5) / (T(1) - dc);
+  if constexpr (SPLIT == 3) return T(0.5) * recip(T(1) - dc);
   else return T(0.5) * rg;
 }
 template <typename T, int SPLIT>
