@@ -15,7 +15,7 @@
 //                                     stage of src/discrete_operators.py:18-101
 //   k_wind_e2c / k_wind_c2e           duo-grid vector ghost fill (src/interpolation.py:347-532)
 //   k_wind_avg                        time-averaged winds (src/averaged_velocity.py:14-62)
-//   k_settle / k_finalize / k_clear_corr, k_diag / k_diag_final   state read-out and diagnostics
+//   k_settle, k_fold_values / k_finalize, k_diag / k_diag_final   state read-out and diagnostics
 // The fused step kernel lives in csadv_step.hpp (instantiated by step_<dtype>_r<recon>.hip), the
 // general step in csadv_general.hpp (general_<dtype>_s<split>.hip), the host-side planning in
 // csadv_plan.cpp.
@@ -248,8 +248,7 @@ __device__ __forceinline__ void ghost_cells(const Solve &S, double *red, int blk
   if (lead) ctl[2] = steps;
 }
 
-// Add the last step's partials to the correction total (once; used by finalize and the
-// diagnostics).
+// Add the last step's partials to the correction total (once; used by the full ghost fill).
 __global__ void k_settle(Solve *solves, int first) {
   __shared__ double red[BLOCK];
   Solve &S = solves[first + blockIdx.x];
@@ -263,6 +262,17 @@ __global__ void k_settle(Solve *solves, int first) {
   }
   __syncthreads();
   if (threadIdx.x == 0) D.ctl[3] = 0;
+}
+
+// The correction total of a tracer, the pending partials added for this block alone.
+__device__ __forceinline__ double settled_total(const Solve &S, int tr) {
+  __shared__ double red[BLOCK];
+  const csadv_solve_desc &D = S.d;
+  if (D.mf != 3 || !D.corr) return 0.0;
+  const int steps = D.ctl[1], pending = D.ctl[3];
+  const double c0 = D.corr[tr], c1 = D.corr[D.ntr + tr];
+  const double sum = pending ? partial_sum(D.partials + (int64_t)tr * S.part_per_tracer, S.part_per_tracer, red) : 0.0;
+  return corr_total(D.dt, D.a2, c0, c1, sum, pending, steps);
 }
 
 // A handle of several solves: workgroup b takes item b of the ghost work list (ghost_list).
@@ -281,40 +291,56 @@ __global__ __launch_bounds__(BLOCK) void k_ghost1(const Solve one) {
   ghost_cells<T>(one, red, blockIdx.x == gridDim.x - 1 ? -1 : (int)blockIdx.x, (int)blockIdx.z);
 }
 
-// Fold the correction totals (interior) and the FP32 state offsets (every cell: a ghost value is
-// a weighted sum with weights summing to 1, so it takes the offset as it is) into the current
-// buffer; k_clear_corr then clears them.
-template <typename T>
-__global__ void k_finalize(Solve *solves, int first) {
-  Solve &S = solves[first + blockIdx.y];
+// csadv_finalize folds the correction totals (interior) and the FP32 state offsets (every cell: a
+// ghost value is a weighted sum with weights summing to 1, so it takes the offset as it is) into the
+// current buffer, in two launches: k_fold_values (one block per solve) settles the totals, moves
+// them with the offsets into fold ([solve][max_tracers][2]) and clears both; k_finalize adds them.
+__global__ __launch_bounds__(BLOCK) void k_fold_values(Solve *solves, int first, double *fold, int max_tracers) {
+  __shared__ double red[BLOCK];
+  Solve &S = solves[first + blockIdx.x];
   csadv_solve_desc &D = S.d;
-  if (D.mf != 3 && !D.offset) return;
-  const int N = D.N, M = S.M, ld = D.ld;
-  T *Q = reinterpret_cast<T *>((D.ctl[1] & 1) ? D.q1 : D.q0);
-  const int64_t tot = (int64_t)6 * M * M, mm = (int64_t)M * M;
+  double *f = fold + (int64_t)blockIdx.x * max_tracers * 2;
+  const int steps = D.ctl[1], pending = D.mf == 3 && D.ctl[3];
   for (int tr = 0; tr < D.ntr; ++tr) {
-    const double cf = D.mf == 3 ? D.corr[(D.ctl[1] & 1) * D.ntr + tr] : 0.0;
-    const double off = D.offset ? D.offset[tr] : 0.0;
-    if (cf == 0.0 && off == 0.0) continue;
-    for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < tot; idx += (int64_t)gridDim.x * blockDim.x) {
-      const int p = (int)(idx / mm);
-      const int rem = (int)(idx - p * mm);
-      const int j = rem / M, i = rem % M;
-      const bool interior = i >= NG && i < N + NG && j >= NG && j < N + NG;
-      if (!interior && off == 0.0) continue;
-      T &v = Q[tr * S.tstride + p * S.pstride + (int64_t)j * ld + i];
-      const double c = interior ? cf * D.gc64[(int64_t)j * ld + i] : 0.0;
-      v = (T)(((double)v + off) + c);
-    }
+    const double sum = pending ? partial_sum(D.partials + (int64_t)tr * S.part_per_tracer, S.part_per_tracer, red) : 0.0;
+    if (threadIdx.x != 0) continue;
+    f[2 * tr] = D.mf == 3 ? corr_total(D.dt, D.a2, D.corr[tr], D.corr[D.ntr + tr], sum, pending, steps) : 0.0;
+    f[2 * tr + 1] = D.offset ? D.offset[tr] : 0.0;
+    if (D.mf == 3) D.corr[tr] = D.corr[D.ntr + tr] = 0.0;
+    if (D.offset) D.offset[tr] = 0.0;
   }
+  __syncthreads();                     // every thread has read the flag
+  if (threadIdx.x == 0 && pending) D.ctl[3] = 0;
 }
 
-__global__ void k_clear_corr(Solve *solves, int first) {
-  csadv_solve_desc &D = solves[first + blockIdx.x].d;
-  if (D.mf == 3)
-    for (int k = threadIdx.x; k < 2 * D.ntr; k += blockDim.x) D.corr[k] = 0.0;
-  if (D.offset)
-    for (int k = threadIdx.x; k < D.ntr; k += blockDim.x) D.offset[k] = 0.0;
+// One wavefront per row of a panel; grid: x = blocks of BLOCK / WAVE rows of the 6 panels (strided),
+// y = tracer, z = solve.  (With a flat index over all cells, two 64-bit divisions each and the tracers
+// one after another it took 41 us on average over 64 FP32 solves of up to N = 512.)
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void k_finalize(Solve *solves, int first, const double *fold, int max_tracers) {
+#pragma clang fp contract(off)
+  const Solve &S = solves[first + blockIdx.z];
+  const csadv_solve_desc &D = S.d;
+  const int tr = blockIdx.y;
+  if (tr >= D.ntr) return;
+  const double *f = fold + ((int64_t)blockIdx.z * max_tracers + tr) * 2;
+  const double cf = f[0], off = f[1];
+  if (cf == 0.0 && off == 0.0) return;
+  const int M = S.M, ld = D.ld, iend = D.N + NG, lane = threadIdx.x & (WAVE - 1);
+  T *Q = reinterpret_cast<T *>((D.ctl[1] & 1) ? D.q1 : D.q0) + tr * S.tstride;
+  for (int r = blockIdx.x * (BLOCK / WAVE) + threadIdx.x / WAVE; r < 6 * M; r += gridDim.x * (BLOCK / WAVE)) {
+    const int p = r / M, j = r - p * M;
+    const bool row_in = j >= NG && j < iend;
+    if (!row_in && off == 0.0) continue;
+    T *q = Q + p * S.pstride + (int64_t)j * ld;
+    const double *g = D.gc64 + (int64_t)j * ld;
+    for (int i = lane; i < M; i += WAVE) {
+      const bool interior = row_in && i >= NG && i < iend;
+      if (!interior && off == 0.0) continue;
+      const double c = interior ? cf * g[i] : 0.0;
+      q[i] = (T)(((double)q[i] + off) + c);
+    }
+  }
 }
 
 // ------------------------------------------------------------------ MF-AF on the fused step
@@ -418,7 +444,7 @@ __global__ void k_remap_latlon(const Solve *solves, int solve, int tracer, const
   const double pi = 3.141592653589793, a = pi * 0.5 * 0.5, dx = 2.0 * a / N;
   const double lon_step = (pi - (-pi)) / (nlon - 1), lat_step = (pi * 0.5 - (-pi * 0.5)) / (nlat - 1);
   const T *Q = reinterpret_cast<const T *>((D.ctl[1] & 1) ? D.q1 : D.q0) + tracer * S.tstride;
-  const double cf = (D.corr && D.mf == 3) ? D.corr[(D.ctl[1] & 1) * D.ntr + tracer] : 0.0;
+  const double cf = field ? 0.0 : settled_total(S, tracer);
   const double off = D.offset ? D.offset[tracer] : 0.0;
   const int64_t total = (int64_t)nlon * nlat;
   for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < total; k += (int64_t)gridDim.x * blockDim.x) {
@@ -695,21 +721,24 @@ __device__ __forceinline__ void kmerge(KSum &a, const KSum &b) {
   a.c += b.c;
 }
 
-// Butterfly reductions over the 64 lanes of a wavefront (cross-lane shuffles, no LDS): lane 0
+// Reductions over the 64 lanes of a wavefront by lane swaps and DPP shifts (warp_sum's moves): lane 0
 // ends with the wavefront's total, combined in a fixed order.
+template <typename F> __device__ __forceinline__ void wave_reduce(F step) {
+  step([](double v) { return lane_up32(v); });
+  step([](double v) { return lane_up16(v); });
+  step([](double v) { return dpp_move<0x108>(v); });
+  step([](double v) { return dpp_move<0x104>(v); });
+  step([](double v) { return dpp_move<0x102>(v); });
+  step([](double v) { return dpp_move<0x101>(v); });
+}
 __device__ __forceinline__ void wave_ksum(KSum &a) {
-  for (int off = WAVE / 2; off > 0; off >>= 1) {
-    const KSum b{__shfl_xor(a.s, off, WAVE), __shfl_xor(a.c, off, WAVE)};
+  wave_reduce([&](auto up) {
+    const KSum b{up(a.s), up(a.c)};
     kmerge(a, b);
-  }
+  });
 }
 __device__ __forceinline__ double wave_max(double v) {
-  for (int off = WAVE / 2; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, WAVE));
-  return v;
-}
-
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
+  wave_reduce([&](auto up) { v = fmax(v, up(v)); });
   return v;
 }
 
@@ -723,7 +752,7 @@ __device__ __forceinline__ void diag_block(KSum m, KSum a1, KSum a2, double mx, 
   wave_ksum(a1);
   wave_ksum(a2);
   mx = wave_max(mx);
-  nan = wave_sum(nan);
+  nan = warp_sum(nan);
   const int w = threadIdx.x / WAVE;
   if ((threadIdx.x & (WAVE - 1)) == 0) {
     red[w][0] = m.s; red[w][1] = m.c; red[w][2] = a1.s; red[w][3] = a1.c;
@@ -747,8 +776,9 @@ __device__ __forceinline__ void diag_block(KSum m, KSum a1, KSum a2, double mx, 
 // Diagnostics of tracers tracer0 .. tracer0 + gridDim.y - 1 of one solve (grid: kDiagBlocks x
 // tracers): per block the compensated FP64 sums of the mass Q g dx dy (src/diagnostics.py:14-26)
 // and of |e| and e^2, and the max |e| (src/errors.py:99-113), with e = qexact - Q when the exact
-// field is given ([tracers][6][N][N] FP64) and e = Q otherwise.  Q = S + C g (the pending
-// mass-fixer total; + the FP32 state offset), read from the solve's current buffer.
+// field is given ([tracers][6][N][N] FP64) and e = Q otherwise.  Q = S + C g (+ the FP32 state
+// offset), read from the solve's current buffer; every block settles the mass-fixer total C for
+// itself, in the one order of partial_sum.
 template <typename T>
 __global__ __launch_bounds__(BLOCK) void k_diag(const Solve *solves, int solve, int tracer0, const double *qex,
                                                 double *part) {
@@ -758,17 +788,16 @@ __global__ __launch_bounds__(BLOCK) void k_diag(const Solve *solves, int solve, 
   const int N = D.N, ld = D.ld;
   const int cur = D.ctl[1] & 1;
   const T *Q = reinterpret_cast<const T *>(cur ? D.q1 : D.q0) + tr * S.tstride;
-  const double cf = (D.corr && D.mf == 3) ? D.corr[cur * D.ntr + tr] : 0.0;
+  const double cf = settled_total(S, tr);
   const double off = D.offset ? D.offset[tr] : 0.0;
   const double dxdy = D.dx * D.dy;
-  const int64_t cells = (int64_t)6 * N * N, nn = (int64_t)N * N;
+  const unsigned cells = 6u * N * N;                 // (N <= 8192: under 2^32)
   const double *qe = qex ? qex + (int64_t)blockIdx.y * cells : nullptr;
   KSum m{0.0, 0.0}, a1{0.0, 0.0}, a2{0.0, 0.0};
   double mx = 0.0, nan = 0.0;
-  for (int64_t idx = blockIdx.x * (int64_t)BLOCK + threadIdx.x; idx < cells; idx += (int64_t)gridDim.x * BLOCK) {
-    const int p = (int)(idx / nn);
-    const int rem = (int)(idx - p * nn);
-    const int j = rem / N + NG, i = rem % N + NG;
+  for (unsigned idx = blockIdx.x * BLOCK + threadIdx.x; idx < cells; idx += gridDim.x * BLOCK) {
+    const unsigned row = idx / (unsigned)N, p = row / (unsigned)N;
+    const int i = (int)(idx - row * N) + NG, j = (int)(row - p * N) + NG;
     const double g = D.gc64[(int64_t)j * ld + i];
     const double q = ((double)Q[p * S.pstride + (int64_t)j * ld + i] + off) + cf * g;
     kadd(m, q * g * dxdy);
@@ -1056,6 +1085,7 @@ int csadv_create(const csadv_solve_desc *solves, int32_t nsolve, int32_t tile, c
   if ((e = hipMalloc(&h->dev, sizeof(Solve) * nsolve)) != hipSuccess ||
       (e = hipMalloc(&h->qsets, sizeof(FieldSet) * nsolve)) != hipSuccess ||
       (e = hipMalloc(&h->wsets, sizeof(FieldSet) * nsolve)) != hipSuccess ||
+      (e = hipMalloc(&h->fold, sizeof(double) * 2 * maxtr * nsolve)) != hipSuccess ||
       (e = hipMalloc(&h->red, sizeof(double) * diag_scratch_words(maxtr))) != hipSuccess)
     return fail(h, CSADV_E_HIP, std::string("descriptor allocation: ") + hipGetErrorString(e));
   return csadv_update(h, solves, nsolve, nullptr);
@@ -1238,12 +1268,10 @@ int diag_args(csadv_t *h, int solve, int tracer0, int ntracers, double limit, co
   return CSADV_OK;
 }
 
-// k_settle (the pending mass-fixer total), the block partials into scratch (diag_scratch_words
-// doubles for ntracers) and the totals into out ([ntracers][4] device doubles); no host
+// The block partials into scratch (diag_scratch_words doubles for ntracers) and the totals into out ([ntracers][4] device doubles); no host
 // synchronisation and no allocation, so a graph may capture it.
 int diagnostics(csadv_t *h, int solve, int tracer0, int ntracers, const double *qexact, double limit, double *out,
                 double *scratch, hipStream_t st) {
-  hipLaunchKernelGGL(k_settle, dim3(1), dim3(BLOCK), 0, st, h->dev, solve);
   if (h->dtype == CSADV_F64)
     hipLaunchKernelGGL(k_diag<double>, dim3(kDiagBlocks, ntracers), dim3(BLOCK), 0, st, h->dev, solve, tracer0, qexact,
                        scratch);
@@ -1376,12 +1404,20 @@ int csadv_finalize(csadv_t *h, int32_t solve, void *stream) {
   const int ns = (int)h->desc.size();
   if (solve < -1 || solve >= ns) return fail(h, CSADV_E_ARG, "finalize: bad solve index");
   const int first = solve < 0 ? 0 : solve, count = solve < 0 ? ns : 1;
-  hipLaunchKernelGGL(k_settle, dim3(count), dim3(BLOCK), 0, st, h->dev, first);
+  int maxM = 0, maxtr = 0;             // of the solves that have anything to fold
+  for (int s = first; s < first + count; ++s) {
+    const csadv_solve_desc &d = h->desc[s];
+    if (d.mf != 3 && !d.offset) continue;
+    maxM = std::max(maxM, h->host[s].M);
+    maxtr = std::max(maxtr, d.ntr);
+  }
+  if (!maxtr) return CSADV_OK;
+  hipLaunchKernelGGL(k_fold_values, dim3(count), dim3(BLOCK), 0, st, h->dev, first, h->fold, h->red_tracers);
+  const dim3 grid(std::min(1024, (6 * maxM + BLOCK / WAVE - 1) / (BLOCK / WAVE)), maxtr, count);
   if (h->dtype == CSADV_F64)
-    hipLaunchKernelGGL(k_finalize<double>, dim3(256, count), dim3(BLOCK), 0, st, h->dev, first);
+    hipLaunchKernelGGL(k_finalize<double>, grid, dim3(BLOCK), 0, st, h->dev, first, h->fold, h->red_tracers);
   else
-    hipLaunchKernelGGL(k_finalize<float>, dim3(256, count), dim3(BLOCK), 0, st, h->dev, first);
-  hipLaunchKernelGGL(k_clear_corr, dim3(count), dim3(64), 0, st, h->dev, first);
+    hipLaunchKernelGGL(k_finalize<float>, grid, dim3(BLOCK), 0, st, h->dev, first, h->fold, h->red_tracers);
   HIPCHK(h, hipGetLastError());
   return CSADV_OK;
 }
@@ -1442,7 +1478,6 @@ int csadv_remap_latlon(csadv_t *h, int32_t solve, int32_t tracer, const double *
   if (nlat < 2 || nlon < 2 || (int64_t)nlat * nlon > ((int64_t)1 << 31))
     return fail(h, CSADV_E_RANGE, "remap: nlat, nlon must be >= 2 and nlat * nlon <= 2^31");
   hipStream_t st = (hipStream_t)stream;
-  if (!field) hipLaunchKernelGGL(k_settle, dim3(1), dim3(BLOCK), 0, st, h->dev, solve);   // totals current
   const int blocks = (int)std::min<int64_t>(4096, ((int64_t)nlat * nlon + BLOCK - 1) / BLOCK);
   if (h->dtype == CSADV_F64)
     hipLaunchKernelGGL(k_remap_latlon<double>, dim3(blocks), dim3(BLOCK), 0, st, h->dev, solve, tracer, field, nlat,
@@ -1597,6 +1632,7 @@ void csadv_destroy(csadv_t *h) {
   if (h->qsets) (void)hipFree(h->qsets);
   if (h->wsets) (void)hipFree(h->wsets);
   if (h->red) (void)hipFree(h->red);
+  if (h->fold) (void)hipFree(h->fold);
   for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
   drop_graph(h);
   if (h->cap) (void)hipStreamDestroy(h->cap);

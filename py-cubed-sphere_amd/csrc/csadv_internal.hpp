@@ -40,6 +40,7 @@ struct csadv_s {
   std::vector<SelfSide> sides;    // self: the ghost sources of the 24 panel sides
   std::vector<void *> ftab;       // the bound flux tables, one per solve (null: none)
   double *red = nullptr;          // diagnostics scratch: partials and outputs (diag_scratch_words)
+  double *fold = nullptr;         // csadv_finalize: [solve][red_tracers][2] totals and offsets
   int red_tracers = 1;            // tracers the diagnostics scratch holds (the largest ntr)
   std::vector<int> done;          // host copy of the steps completed per solve (ctl[1])
   std::vector<hipEvent_t> ev;     // profiling event pairs (start, end) around the step kernel
