@@ -5,8 +5,9 @@
  *
  * Every state buffer is device memory owned by the caller (PyTorch tensors on the
  * host side); the library keeps non-owning pointers to it and never frees it.  The
- * library allocates only its own small descriptor tables, in csadv_create; a step
- * neither allocates nor synchronises the stream.  All entry points return
+ * library allocates its own descriptor tables, scratch of some MB at most and, for a small
+ * multi-tracer solve on the general step, work buffers of up to four wavefronts' worth per SIMD
+ * (csadv_create, csadv_update); a step neither allocates nor synchronises the stream.  All entry points return
  * 0 on success and a negative CSADV_E* code on failure; the message of the last
  * failure of a handle is returned by csadv_last_error().  Handles are not
  * thread-safe; independent handles are.

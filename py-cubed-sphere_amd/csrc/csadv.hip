@@ -347,7 +347,7 @@ __global__ __launch_bounds__(BLOCK) void k_finalize(Solve *solves, int first, co
 // The fused step updates every cell with its own second-pass fluxes and, with MF-AF, keeps the
 // fluxes through the 24 panel sides in work ([tracer][panel][E, W, N, S][N]); this kernel
 // replaces them by the cube-edge averages in the boundary cells of the new state (af_fix_cell).
-// grid: x = boundary cells of the 6 panels, y = solve, z = tracer.
+// grid: x = the 6 panels' boundary cells (the largest solve's), y = solve, z = tracer.
 template <typename T>
 __global__ __launch_bounds__(BLOCK) void k_af_fix(const Solve *solves) {
   const Solve &S = solves[blockIdx.y];
@@ -356,17 +356,19 @@ __global__ __launch_bounds__(BLOCK) void k_af_fix(const Solve *solves) {
   if (D.mf != 2 || tr >= D.ntr) return;
   const int run = D.ctl[2];                 // the step k_ghost started (< 0: the solve is halted)
   if (run < 0 || (D.stop > 0 && run >= D.stop)) return;
-  af_fix_cell<T>(S, tr, run, reinterpret_cast<const T *>(D.work) + (int64_t)tr * 24 * D.N, blockIdx.x * BLOCK + threadIdx.x);
+  af_fix_cell<T>(S, tr, run, reinterpret_cast<const T *>(D.work) + (int64_t)tr * 24 * D.N,
+                 [&](int p, int side) { return af_side(D.orient + (p * 4 + side) * 7, side, D.N); });
 }
 
 // A handle of one solve whose steps fill their own ghosts: step k of the running sequence (the
 // completed steps, ctl[1], stand still until its end).  grid: x = boundary cells, y = tracer.
 template <typename T>
-__global__ __launch_bounds__(BLOCK) void k_af_fix1(const Solve one, int k) {
+__global__ __launch_bounds__(BLOCK) void k_af_fix1(const Solve one, const AfSides af, int k) {
   const csadv_solve_desc &D = one.d;
   const int tr = blockIdx.y, run = D.ctl[1] + k;
   if (D.ctl[0] || (D.stop > 0 && run >= D.stop)) return;
-  af_fix_cell<T>(one, tr, run, reinterpret_cast<const T *>(D.work) + (int64_t)tr * 24 * D.N, blockIdx.x * BLOCK + threadIdx.x);
+  af_fix_cell<T>(one, tr, run, reinterpret_cast<const T *>(D.work) + (int64_t)tr * 24 * D.N,
+                 [&](int p, int side) { return af.side[p * 4 + side]; });
 }
 
 // End of a sequence of n steps that filled their own ghosts: the last executed step's mass-fixer
@@ -950,6 +952,43 @@ int wind_avg(csadv_t *h, hipStream_t st, bool all, int k = 0) {
   return CSADV_OK;
 }
 
+// The MF-AF sides of every solve that has them (AfSides), from the solves' orientation tables.
+int plan_af(csadv_t *h, hipStream_t st) {
+  h->af.assign(h->host.size(), AfSides{});
+  for (size_t s = 0; s < h->host.size(); ++s) {
+    const csadv_solve_desc &d = h->desc[s];
+    if (d.mf != 2) continue;
+    int32_t o[24 * 7];
+    HIPCHK(h, hipMemcpyAsync(o, d.orient, sizeof(o), hipMemcpyDeviceToHost, st));
+    HIPCHK(h, hipStreamSynchronize(st));
+    for (int t = 0; t < 24; ++t) h->af[s].side[t] = af_side(o + 7 * t, t & 3, d.N);
+  }
+  return CSADV_OK;
+}
+
+// Tracers per launch of the general step, and the work buffers of the largest group (one group
+// runs at a time).  Without the memory for them the tracers go one by one.
+int plan_general(csadv_t *h) {
+  h->gp_group.clear();
+  int64_t need = 0;
+  for (const Solve &S : h->host) {
+    h->gp_group.push_back(gp_group(S));
+    if (h->gp_group.back() > 1) need = std::max(need, h->gp_group.back() * gp_work_stride(S.d));
+  }
+  if (need > h->gp_work_bytes) {
+    if (h->gp_work) (void)hipFree(h->gp_work);
+    h->gp_work = nullptr;
+    h->gp_work_bytes = 0;
+    if (hipMalloc(&h->gp_work, need) == hipSuccess) {
+      h->gp_work_bytes = need;
+    } else {
+      (void)hipGetLastError();
+      h->gp_group.assign(h->host.size(), 1);
+    }
+  }
+  return CSADV_OK;
+}
+
 // Whether the steps of the handle fill their own ghosts (self_fill), with two buffers for the mass-
 // fixer partials of alternating steps.
 int plan_self(csadv_t *h, hipStream_t st) {
@@ -1032,6 +1071,9 @@ int upload_plan(csadv_t *h, hipStream_t st) {
   }
   HIPCHK(h, hipMemcpyAsync(h->dev, h->host.data(), sizeof(Solve) * nsolve, hipMemcpyHostToDevice, st));
   HIPCHK(h, hipStreamSynchronize(st));   // the lists above are host memory of this call
+  const int rc = plan_af(h, st);
+  if (rc) return rc;
+  if (h->general) return plan_general(h);
   return plan_self(h, st);
 }
 
@@ -1310,14 +1352,14 @@ int enqueue_step(csadv_t *h, hipStream_t st, bool allow_prof, int k, int n) {
     ++h->ev_used;
   }
   if (h->mfaf && self) {
-    const dim3 grid((6 * 4 * (h->desc[0].N - 1) + BLOCK - 1) / BLOCK, h->desc[0].ntr);
-    if (h->dtype == CSADV_F64) hipLaunchKernelGGL(k_af_fix1<double>, grid, dim3(BLOCK), 0, st, h->host[0], k);
-    else hipLaunchKernelGGL(k_af_fix1<float>, grid, dim3(BLOCK), 0, st, h->host[0], k);
+    const dim3 grid(6 * af_blocks(h->desc[0].N), h->desc[0].ntr);
+    if (h->dtype == CSADV_F64) hipLaunchKernelGGL(k_af_fix1<double>, grid, dim3(BLOCK), 0, st, h->host[0], h->af[0], k);
+    else hipLaunchKernelGGL(k_af_fix1<float>, grid, dim3(BLOCK), 0, st, h->host[0], h->af[0], k);
     HIPCHK(h, hipGetLastError());
   } else if (h->mfaf) {   // MF-AF: the cube-edge flux averages into the boundary cells
     int maxN = 0, maxtr = 1;
     for (auto &d : h->desc) { maxN = std::max(maxN, d.N); maxtr = std::max(maxtr, d.ntr); }
-    const dim3 grid((6 * 4 * (maxN - 1) + BLOCK - 1) / BLOCK, (int)h->desc.size(), maxtr);
+    const dim3 grid(6 * af_blocks(maxN), (int)h->desc.size(), maxtr);
     if (h->dtype == CSADV_F64) hipLaunchKernelGGL(k_af_fix<double>, grid, dim3(BLOCK), 0, st, h->dev);
     else hipLaunchKernelGGL(k_af_fix<float>, grid, dim3(BLOCK), 0, st, h->dev);
     HIPCHK(h, hipGetLastError());
@@ -1633,6 +1675,7 @@ void csadv_destroy(csadv_t *h) {
   if (h->wsets) (void)hipFree(h->wsets);
   if (h->red) (void)hipFree(h->red);
   if (h->fold) (void)hipFree(h->fold);
+  if (h->gp_work) (void)hipFree(h->gp_work);
   for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
   drop_graph(h);
   if (h->cap) (void)hipStreamDestroy(h->cap);

@@ -32,7 +32,7 @@ __device__ __forceinline__ void halo_src(const int32_t *o, int d, int r, int &q,
 
 // Side of the neighbour across (p, side) and the sign relating the two axes across the edge.
 // o = orient row {q, ib, id, ir, jb, jd, jr}; sides 0 E, 1 W, 2 N, 3 S.
-__device__ __forceinline__ void across(const int32_t *o, int side, int &sq, int &sign) {
+__host__ __device__ inline void across(const int32_t *o, int side, int &sq, int &sign) {
   const int id = o[2], jd = o[5];
   sq = (id > 0) + (id == 0) * (2 + (jd > 0));       // id > 0: W; id < 0: E; id == 0: jd > 0 S, else N
   const int out = (side == 0 || side == 2) ? 1 : -1;
@@ -455,35 +455,49 @@ __device__ __forceinline__ double fabs_t(double v) { return fabs(v); }
 // (their fluxes leave the cell there) and (f_avg - f) / g at the west and south sides.  Item idx
 // is one boundary cell of a panel (4 (N - 1) of them per panel), so a corner cell takes both of
 // its sides' differences in one fixed order; run is the step that produced the state.
-template <typename T>
-__device__ __forceinline__ T af_average(const T *F, const int32_t *orient, int N, int p, int side, int k) {
-  const T own = F[(p * 4 + side) * N + k];
-  const int32_t *o = orient + (p * 4 + side) * 7;
-  int q, i, j, sq, sign;
-  halo_src(o, 0, k + NG, q, i, j);
+// Where the flux across (panel, side) at position k lies: index a + k b of F, and the sign.
+struct AfSide {
+  int32_t a, b, sign;
+};
+__host__ __device__ inline AfSide af_side(const int32_t *o, int side, int N) {
+  // o: the side's orientation row {q, ib, id, ir, jb, jd, jr}, here at depth 0 and row k + NG
+  int sq, sign;
   across(o, side, sq, sign);
-  const T nb = F[(q * 4 + sq) * N + (sq < 2 ? j : i) - NG];
-  return T(0.5) * own + T(0.5) * (sign > 0 ? nb : -nb);
+  const int along0 = sq < 2 ? o[4] + o[6] * NG : o[1] + o[3] * NG;
+  return {(o[0] * 4 + sq) * N + along0 - NG, sq < 2 ? o[6] : o[3], sign};
 }
 
-template <typename T>
-__device__ __forceinline__ void af_fix_cell(const Solve &S, int tr, int run, const T *F, int idx) {
+struct AfSides {
+  AfSide side[24];
+};
+
+// The grid's x covers the panels' rings, panel by panel (af_blocks blocks each), so that the panel is
+// wave-uniform and its sides' places are scalar loads.  side_of(p, side): the AfSide of a panel side,
+// from the orientation table or from kernel arguments (a chain of loads less).
+inline int af_blocks(int N) { return (4 * (N - 1) + BLOCK - 1) / BLOCK; }
+template <typename T, typename SideOf>
+__device__ __forceinline__ void af_fix_cell(const Solve &S, int tr, int run, const T *F, SideOf side_of) {
   const csadv_solve_desc &D = S.d;
   const int N = D.N, ld = D.ld, i0 = NG, iend = N + NG;
-  const int ring = 4 * (N - 1);
-  if (idx >= 6 * ring) return;
-  const int p = idx / ring, c = idx - p * ring;
-  // ring order: south row, north row, west column, east column (corners in the rows)
+  const int per = gridDim.x / 6, p = blockIdx.x / per, c = (blockIdx.x - p * per) * BLOCK + threadIdx.x;
+  const AfSide sides[4] = {side_of(p, 0), side_of(p, 1), side_of(p, 2), side_of(p, 3)};
+  if (c >= 4 * (N - 1)) return;
   int i, j;
+  // ring order: south row, north row, west column, east column (corners in the rows)
   if (c < N) { i = i0 + c; j = i0; }
   else if (c < 2 * N) { i = i0 + c - N; j = iend - 1; }
   else if (c < 3 * N - 2) { i = i0; j = i0 + 1 + c - 2 * N; }
   else { i = iend - 1; j = i0 + 1 + c - (3 * N - 2); }
+  const auto average = [&](int side, int k) {
+    const AfSide f = sides[side];
+    const T own = F[(p * 4 + side) * N + k], nb = F[f.a + f.b * k];
+    return T(0.5) * own + T(0.5) * (f.sign > 0 ? nb : -nb);
+  };
   T d = T(0);
-  if (i == iend - 1) d += F[(p * 4 + 0) * N + j - NG] - af_average(F, D.orient, N, p, 0, j - NG);
-  if (i == i0) d += af_average(F, D.orient, N, p, 1, j - NG) - F[(p * 4 + 1) * N + j - NG];
-  if (j == iend - 1) d += F[(p * 4 + 2) * N + i - NG] - af_average(F, D.orient, N, p, 2, i - NG);
-  if (j == i0) d += af_average(F, D.orient, N, p, 3, i - NG) - F[(p * 4 + 3) * N + i - NG];
+  if (i == iend - 1) d += F[(p * 4 + 0) * N + j - NG] - average(0, j - NG);
+  if (i == i0) d += average(1, j - NG) - F[(p * 4 + 1) * N + j - NG];
+  if (j == iend - 1) d += F[(p * 4 + 2) * N + i - NG] - average(2, i - NG);
+  if (j == i0) d += average(3, i - NG) - F[(p * 4 + 3) * N + i - NG];
   T *Q = reinterpret_cast<T *>(((run + 1) & 1) ? D.q1 : D.q0) + tr * S.tstride + p * S.pstride;
   const T rg = reinterpret_cast<const T *>(D.rgc)[(int64_t)j * ld + i];
   Q[(int64_t)j * ld + i] += d * rg;

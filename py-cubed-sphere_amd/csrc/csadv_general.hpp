@@ -1,12 +1,12 @@
 // General step: ET-S72 and ET-PL07, whose halo is the adjacent panels' own cells (the copy halo
 // of src/interpolation.py:320-340 and src/halo_data.py) rather than the duo-grid interpolation,
-// as two marched passes per tracer (src/discrete_operators.py:18-101):
+// as two marched passes, some tracers at once (src/discrete_operators.py:18-101):
 //
 //   pass 1: x- and y-fluxes of Q, the split half-steps Qx and Qy of every interior cell;
 //   pass 2: x-fluxes of Qy, y-fluxes of Qx, and the update of Q (MF-0, MF-AF), or the
 //           divergence and its partial sums (MF-PR);
 //   MF-AF: k_gp_af_fix puts the cube-edge flux averages into the boundary cells;
-//   MF-PR: k_gp_prsum sums the partials, k_gp_update applies the projection and the update.
+//   MF-PR: k_gp_update sums the partials and applies the projection and the update.
 //
 // Each pass marches one wavefront down a column strip as the fused step does (lane = column,
 // the 3-cell halo in the outer lanes, x windows by DPP, register rings for the y windows).  No
@@ -423,7 +423,7 @@ __device__ __forceinline__ bool gp_running(const csadv_solve_desc &D, int run) {
 }
 
 template <typename T, int RECON, bool RK2, int PASS, int SPLIT>
-__device__ __forceinline__ void gp_item(const Solve &S, int tr, int p, int sx, int sg, bool last) {
+__device__ __forceinline__ void gp_item(const Solve &S, T *work, int tr, int p, int sx, int sg, bool last) {
   const csadv_solve_desc &D = S.d;
   const int lane = threadIdx.x;
   int run;
@@ -439,7 +439,6 @@ __device__ __forceinline__ void gp_item(const Solve &S, int tr, int p, int sx, i
   const int nx = min(S.strip_w, iend - ti), ny = min(S.seg_l, iend - tj);
   const int ps = (int)S.pstride;
   const WorkLayout w = work_layout(N, ld, D.ldu);
-  T *work = reinterpret_cast<T *>(D.work);
   const bool odd = run & 1;                   // the state of step n lives in q[n & 1]
   const int64_t toff = tr * S.tstride;
   T *qin = reinterpret_cast<T *>(odd ? D.q1 : D.q0) + toff, *qout = reinterpret_cast<T *>(odd ? D.q0 : D.q1) + toff;
@@ -516,57 +515,67 @@ __device__ __forceinline__ void gp_item(const Solve &S, int tr, int p, int sx, i
   }
 }
 
-// One tracer's pass of one solve; the descriptor travels in the kernel arguments.  last: this
-// pass ends the step (pass 2 of the last tracer with neither MF-AF nor MF-PR after it).
+// The work buffers of the tracers of one launch: tracer tr0 + blockIdx.y uses the blockIdx.y-th of
+// them, `stride` bytes apart.
+struct GpWork {
+  char *base;
+  int64_t stride;
+  int tr0;
+};
+template <typename T> __device__ __forceinline__ T *gp_work(const GpWork &w) {
+  return reinterpret_cast<T *>(w.base + blockIdx.y * w.stride);
+}
+
+// A pass of some tracers of one solve (grid: items, tracers); the descriptor travels in the kernel
+// arguments.  last: this pass ends the step (pass 2 of the last tracers with neither MF-AF nor MF-PR
+// after it).
 template <typename T, int RECON, bool RK2, int PASS, int SPLIT>
-__global__ __launch_bounds__(WAVE) void k_gp_pass(const Solve one, int tr, int last) {
+__global__ __launch_bounds__(WAVE) void k_gp_pass(const Solve one, const GpWork w, int last) {
   int p, sx, sg;
   if (!gen_item(one, touch_solve(one, blockIdx.x), p, sx, sg)) return;
-  gp_item<T, RECON, RK2, PASS, SPLIT>(one, tr, p, sx, sg, last != 0);
+  gp_item<T, RECON, RK2, PASS, SPLIT>(one, gp_work<T>(w), w.tr0 + blockIdx.y, p, sx, sg,
+                                      last != 0 && blockIdx.y == gridDim.y - 1);
 }
 
 // MF-AF: the cube-edge averages of the second pass's fluxes into the boundary cells of the new
-// state (af_fix_cell).  grid: boundary cells of the 6 panels.
+// state (af_fix_cell).  grid: boundary cells of the 6 panels, tracers.
 template <typename T>
-__global__ __launch_bounds__(BLOCK) void k_gp_af_fix(const Solve one, int tr, int last) {
+__global__ __launch_bounds__(BLOCK) void k_gp_af_fix(const Solve one, const GpWork w, const AfSides af, int last) {
   const csadv_solve_desc &D = one.d;
   const int run = D.ctl[2];
   if (!gp_running(D, run)) return;
-  if (last && blockIdx.x == 0 && threadIdx.x == 0) D.ctl[1] = run + 1;
-  const WorkLayout w = work_layout(D.N, D.ld, D.ldu);
-  af_fix_cell<T>(one, tr, run, reinterpret_cast<const T *>(D.work) + w.o_side, blockIdx.x * BLOCK + threadIdx.x);
+  if (last && blockIdx.x == 0 && blockIdx.y == gridDim.y - 1 && threadIdx.x == 0) D.ctl[1] = run + 1;
+  const WorkLayout l = work_layout(D.N, D.ld, D.ldu);
+  af_fix_cell<T>(one, w.tr0 + blockIdx.y, run, gp_work<T>(w) + l.o_side,
+                 [&](int p, int side) { return af.side[p * 4 + side]; });
 }
 
 // MF-PR: the sum of div g over all cells, from the nparts wavefront partials in a fixed order
-// (each lane a strided sum, the wavefronts by shuffles, then the four in index order), into the
-// last double of the tail.  One block.
-template <typename T>
-__global__ __launch_bounds__(BLOCK) void k_gp_prsum(const Solve one, int nparts) {
+// (each thread a strided sum, the wavefronts by lane moves, then the four in index order).  Every
+// block of the update forms it for itself: that costs a block about a microsecond, where a kernel
+// of its own before the update cost a launch and its chain of loads.
+__device__ __forceinline__ double gp_total(const double *part, int nparts) {
   __shared__ double red[BLOCK / WAVE];
-  const csadv_solve_desc &D = one.d;
-  if (!gp_running(D, D.ctl[2])) return;
-  const WorkLayout w = work_layout(D.N, D.ld, D.ldu);
-  double *part = reinterpret_cast<double *>(reinterpret_cast<T *>(D.work) + w.o_red);
   double acc = 0.0;
   for (int k = threadIdx.x; k < nparts; k += BLOCK) acc += part[k];
   acc = warp_sum(acc);
   if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = acc;
   __syncthreads();
-  if (threadIdx.x == 0) part[w.n_red - 1] = ((red[0] + red[1]) + red[2]) + red[3];
+  return ((red[0] + red[1]) + red[2]) + red[3];
 }
 
 // MF-PR (src/discrete_operators.py:95-101): Q^{n+1} = Q^n - dt (div - g m0 / a2) on the
-// interior, m0 the sum of div g; one thread per interior cell.
+// interior, m0 the sum of div g; one thread per interior cell (grid: cells, tracers).
 template <typename T>
-__global__ __launch_bounds__(BLOCK) void k_gp_update(const Solve one, int tr, int last) {
+__global__ __launch_bounds__(BLOCK) void k_gp_update(const Solve one, const GpWork gw, int nparts, int last) {
   const csadv_solve_desc &D = one.d;
   const int run = D.ctl[2];
   if (!gp_running(D, run)) return;
-  if (last && blockIdx.x == 0 && threadIdx.x == 0) D.ctl[1] = run + 1;
-  const int N = D.N, ld = D.ld;
+  if (last && blockIdx.x == 0 && blockIdx.y == gridDim.y - 1 && threadIdx.x == 0) D.ctl[1] = run + 1;
+  const int N = D.N, ld = D.ld, tr = gw.tr0 + blockIdx.y;
   const WorkLayout w = work_layout(N, ld, D.ldu);
-  const T *work = reinterpret_cast<const T *>(D.work);
-  const double m0 = reinterpret_cast<const double *>(work + w.o_red)[w.n_red - 1];
+  const T *work = gp_work<T>(gw);
+  const double m0 = gp_total(reinterpret_cast<const double *>(work + w.o_red), nparts);
   const bool odd = run & 1;
   const int64_t toff = tr * one.tstride;
   const T *qin = reinterpret_cast<const T *>(odd ? D.q1 : D.q0) + toff;
@@ -587,26 +596,25 @@ inline int gen_blocks(const Solve &S) { return kXcds * ((S.segs + kXcds - 1) / k
 
 }  // namespace gp
 
-// One step of every solve by the general step: per tracer the two passes, then the mass fixer's
-// kernels; the last kernel of the last tracer advances the step counter.
+// One step of every solve by the general step: per group of tracers the two passes, then the mass fixer's
+// kernels; the last kernel of the last group advances the step counter.
 template <typename T, int R, bool RK2, int SP>
 int enqueue_general_k(csadv_t *h, hipStream_t st) {
   for (size_t s = 0; s < h->host.size(); ++s) {
     const Solve &S = h->host[s];
     const csadv_solve_desc &d = S.d;
-    const int blocks = gp::gen_blocks(S);
-    for (int tr = 0; tr < d.ntr; ++tr) {
-      const int last = tr == d.ntr - 1;
-      hipLaunchKernelGGL((gp::k_gp_pass<T, R, RK2, 1, SP>), dim3(blocks), dim3(WAVE), 0, st, S, tr, 0);
-      hipLaunchKernelGGL((gp::k_gp_pass<T, R, RK2, 2, SP>), dim3(blocks), dim3(WAVE), 0, st, S, tr,
-                         last && d.mf == 1);
+    const int blocks = gp::gen_blocks(S), group = h->gp_group[s];
+    for (int tr = 0; tr < d.ntr; tr += group) {
+      const int n = std::min(group, d.ntr - tr), last = tr + n == d.ntr;
+      const gp::GpWork w{group > 1 ? h->gp_work : static_cast<char *>(d.work), group > 1 ? gp_work_stride(d) : 0, tr};
+      hipLaunchKernelGGL((gp::k_gp_pass<T, R, RK2, 1, SP>), dim3(blocks, n), dim3(WAVE), 0, st, S, w, 0);
+      hipLaunchKernelGGL((gp::k_gp_pass<T, R, RK2, 2, SP>), dim3(blocks, n), dim3(WAVE), 0, st, S, w, last && d.mf == 1);
       if (d.mf == 2) {
-        const int cells = 6 * 4 * (d.N - 1);
-        hipLaunchKernelGGL(gp::k_gp_af_fix<T>, dim3((cells + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, st, S, tr, last);
-      } else if (d.mf == 3) {
-        hipLaunchKernelGGL(gp::k_gp_prsum<T>, dim3(1), dim3(BLOCK), 0, st, S, 6 * S.strips * S.segs);
-        hipLaunchKernelGGL(gp::k_gp_update<T>, dim3(gp_blocks((int64_t)6 * d.N * d.N)), dim3(BLOCK), 0, st, S, tr,
+        hipLaunchKernelGGL(gp::k_gp_af_fix<T>, dim3(6 * af_blocks(d.N), n), dim3(BLOCK), 0, st, S, w, h->af[s],
                            last);
+      } else if (d.mf == 3) {
+        hipLaunchKernelGGL(gp::k_gp_update<T>, dim3(std::min(1024, gp_blocks((int64_t)6 * d.N * d.N)), n), dim3(BLOCK), 0,
+                           st, S, w, 6 * S.strips * S.segs, last);
       }
     }
   }

@@ -32,6 +32,10 @@ struct csadv_s {
   bool rk2 = false;               // dp = 2 (separate upwind-side winds)
   int split = 1;                  // splitting of every solve (its metric treatment follows)
   bool general = false;           // ET-S72 / ET-PL07: the general step
+  std::vector<int> gp_group;      // general step: tracers per launch of each solve
+  char *gp_work = nullptr;        // their work buffers (groups of more than one)
+  int64_t gp_work_bytes = 0;
+  std::vector<AfSides> af;        // MF-AF: the flux across each panel side of each solve
   bool mfaf = false;              // a fused-step solve with MF-AF: k_af_fix after the step kernel
   int mode = kRk1;                // FluxMode of every solve, or kMixed
   bool self = false;              // one solve whose step kernel fills its own ghosts (self_fill)

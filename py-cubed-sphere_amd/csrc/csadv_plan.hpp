@@ -150,6 +150,21 @@ inline int64_t flux_elems(int N, int split) {
   return flux_x_elems(N, split) + (int64_t)6 * (N + 2 * NG + 1) * general_ld(N) * flux_words(split);
 }
 
+// Tracers of one launch of the general step's kernels, each with a work buffer of its own in the
+// handle (gp_work_stride bytes; the caller's holds one tracer and serves where the group is 1): as many
+// as keep a launch under 4 wavefronts per SIMD in FP64 and 12 in FP32.  One tracer at a time leaves the
+// chip idle on small solves: N = 64, 4 tracers, FP64 52.8 -> 15.0 us per step, FP32 68 -> 16.5; N = 384,
+// 3 tracers, 93.8 -> 56.3 and 110 -> 47.  With 12 in FP64, N = 728 with 3 tracers gains nothing (222 us
+// either way), in FP32 181 -> 133.
+inline int64_t gp_work_stride(const csadv_solve_desc &d) {
+  const WorkLayout w = work_layout(d.N, d.ld, d.ldu);
+  return (w.total * (d.dtype == CSADV_F64 ? 8 : 4) + w.n_red * 8 + 255) / 256 * 256;
+}
+inline int gp_group(const Solve &S) {
+  const int g = (S.d.dtype == CSADV_F64 ? 4096 : 12288) / (S.part_per_tracer > 0 ? S.part_per_tracer : 1);
+  return g < 1 ? 1 : g < S.d.ntr ? g : S.d.ntr;
+}
+
 // Elements (of the state's dtype) of the work buffer the fused step needs: MF-AF keeps the
 // second pass's cube-edge fluxes, [ntr][6][4][N]; none otherwise.
 inline int64_t fused_work_elems(const csadv_solve_desc &d) {
