@@ -397,6 +397,16 @@ __global__ __launch_bounds__(BLOCK) void k_advance(const Solve one, int n, const
   }
 }
 
+// The words of every solve that csadv_update reads back (one block per solve).
+__global__ __launch_bounds__(BLOCK) void k_gather_plan(const Solve *solves, PlanWords *out) {
+  const csadv_solve_desc &D = solves[blockIdx.x].d;
+  PlanWords &o = out[blockIdx.x];
+  const int t = threadIdx.x;
+  if (t < 4) o.ctl[t] = D.ctl[t];
+  if (t < 24 * 7) o.orient[t] = D.orient[t];
+  if (t == 0) o.ok = 1;
+}
+
 // Whether the ghost recipes are those of the Lagrange tables in the order the self-filling step
 // reads them (ok stays 1): strips by (panel, side), the depth slowest where the source strip runs
 // along x and fastest elsewhere; corners by (panel, E / W, depth, row).
@@ -952,20 +962,6 @@ int wind_avg(csadv_t *h, hipStream_t st, bool all, int k = 0) {
   return CSADV_OK;
 }
 
-// The MF-AF sides of every solve that has them (AfSides), from the solves' orientation tables.
-int plan_af(csadv_t *h, hipStream_t st) {
-  h->af.assign(h->host.size(), AfSides{});
-  for (size_t s = 0; s < h->host.size(); ++s) {
-    const csadv_solve_desc &d = h->desc[s];
-    if (d.mf != 2) continue;
-    int32_t o[24 * 7];
-    HIPCHK(h, hipMemcpyAsync(o, d.orient, sizeof(o), hipMemcpyDeviceToHost, st));
-    HIPCHK(h, hipStreamSynchronize(st));
-    for (int t = 0; t < 24; ++t) h->af[s].side[t] = af_side(o + 7 * t, t & 3, d.N);
-  }
-  return CSADV_OK;
-}
-
 // Tracers per launch of the general step, and the work buffers of the largest group (one group
 // runs at a time).  Without the memory for them the tracers go one by one.
 int plan_general(csadv_t *h) {
@@ -989,9 +985,9 @@ int plan_general(csadv_t *h) {
   return CSADV_OK;
 }
 
-// Whether the steps of the handle fill their own ghosts (self_fill), with two buffers for the mass-
-// fixer partials of alternating steps.
-int plan_self(csadv_t *h, hipStream_t st) {
+// Whether the steps of the handle may fill their own ghosts (self_fill): the two buffers for the mass-
+// fixer partials of alternating steps, and the check of its recipes queued (its answer in *ok).
+int plan_self(csadv_t *h, int32_t *ok, hipStream_t st) {
   h->self = false;
   if (h->general || h->host.size() != 1 || !self_fill(h->host[0])) return CSADV_OK;
   const Solve &S = h->host[0];
@@ -1001,31 +997,18 @@ int plan_self(csadv_t *h, hipStream_t st) {
     if (h->spart) (void)hipFree(h->spart);
     h->spart = nullptr;
     h->nspart = 0;
-    HIPCHK(h, hipMalloc(&h->spart, sizeof(double) * (2 * n + 1)));
+    HIPCHK(h, hipMalloc(&h->spart, sizeof(double) * 2 * n));
     h->nspart = n;
   }
-  int32_t ok = 1, *flag = reinterpret_cast<int32_t *>(h->spart + 2 * h->nspart);
-  HIPCHK(h, hipMemcpyAsync(flag, &ok, sizeof(ok), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_check_recipes, dim3(32), dim3(BLOCK), 0, st, S, flag);
+  hipLaunchKernelGGL(k_check_recipes, dim3(32), dim3(BLOCK), 0, st, S, ok);
   HIPCHK(h, hipGetLastError());
-  int32_t o[24 * 7];
-  HIPCHK(h, hipMemcpyAsync(&ok, flag, sizeof(ok), hipMemcpyDeviceToHost, st));
-  HIPCHK(h, hipMemcpyAsync(o, S.d.orient, sizeof(o), hipMemcpyDeviceToHost, st));
-  HIPCHK(h, hipStreamSynchronize(st));
-  h->sides.resize(24);
-  for (int t = 0; t < 24; ++t) {
-    const int32_t *r = o + 7 * t;
-    h->sides[t] = {r[0] * (int)S.pstride + r[4] * S.d.ld + r[1], r[5] * S.d.ld + r[2], r[6] * S.d.ld + r[3]};
-  }
-  h->self = ok != 0;
+  h->self = true;
   return CSADV_OK;
 }
 
-// The launch plan of the handle's descriptors and flux tables: each solve's mode, the work lists,
-// and the device copy of all of it.
-int upload_plan(csadv_t *h, hipStream_t st) {
-  const int nsolve = (int)h->host.size();
-  for (int s = 0; s < nsolve; ++s) {
+// Each solve's mode, from its options and its flux table.
+void plan_modes(csadv_t *h) {
+  for (size_t s = 0; s < h->host.size(); ++s) {
     Solve &S = h->host[s];
     const csadv_solve_desc &d = h->desc[s];
     S.mode = own_wind(d) ? kWind : h->ftab[s] ? kTab : d.dp == 2 ? kRk2 : kRk1;
@@ -1036,45 +1019,21 @@ int upload_plan(csadv_t *h, hipStream_t st) {
     }
     h->mode = s == 0 || h->mode == S.mode ? S.mode : (h->rk2 ? kMixed2 : kMixed);
   }
-  // workgroup b runs on XCD b % kXcds (the list interleaves one band of row segments per XCD)
+}
+
+// A work list's device copy (of `n` items before), from host memory that lasts until the caller
+// synchronises the stream.
+int upload_list(csadv_t *h, const std::vector<Item> &list, int4 *&dev, int &n, hipStream_t st) {
   static_assert(sizeof(Item) == sizeof(int4), "work items are read as int4");
-  // (the FP32 multi-solve step kernel marches two tracers per item: kStepGroup in csadv_step.hpp)
-  const int group = (!h->general && h->dtype == CSADV_F32 && nsolve > 1) ? 2 : 1;
-  const std::vector<Item> work = work_list(h->host, group);
-  if ((int)work.size() != h->nwork) {
-    if (h->work) (void)hipFree(h->work);
-    h->work = nullptr;
-    HIPCHK(h, hipMalloc(&h->work, sizeof(int4) * work.size()));
-    h->nwork = (int)work.size();
+  if ((int)list.size() != n) {
+    if (dev) (void)hipFree(dev);
+    dev = nullptr;
+    n = 0;
+    HIPCHK(h, hipMalloc(&dev, sizeof(int4) * list.size()));
+    n = (int)list.size();
   }
-  h->mfaf = false;
-  for (int s = 0; s < nsolve; ++s) h->mfaf = h->mfaf || (!h->general && h->desc[s].mf == 2);
-  HIPCHK(h, hipMemcpyAsync(h->work, work.data(), sizeof(int4) * work.size(), hipMemcpyHostToDevice, st));
-  if (nsolve > 1) {                  // the ghost fill and the winds of a multi-solve handle read their own lists
-    const std::vector<Item> ww = wind_list(h->host, h->nwunsteady);
-    if ((int)ww.size() != h->nwwork) {
-      if (h->wwork) (void)hipFree(h->wwork);
-      h->wwork = nullptr;
-      h->nwwork = 0;
-      HIPCHK(h, hipMalloc(&h->wwork, sizeof(int4) * ww.size()));
-      h->nwwork = (int)ww.size();
-    }
-    HIPCHK(h, hipMemcpyAsync(h->wwork, ww.data(), sizeof(int4) * ww.size(), hipMemcpyHostToDevice, st));
-    const std::vector<Item> gw = ghost_list(h->host);
-    if ((int)gw.size() != h->ngwork) {
-      if (h->gwork) (void)hipFree(h->gwork);
-      h->gwork = nullptr;
-      HIPCHK(h, hipMalloc(&h->gwork, sizeof(int4) * gw.size()));
-      h->ngwork = (int)gw.size();
-    }
-    HIPCHK(h, hipMemcpyAsync(h->gwork, gw.data(), sizeof(int4) * gw.size(), hipMemcpyHostToDevice, st));
-  }
-  HIPCHK(h, hipMemcpyAsync(h->dev, h->host.data(), sizeof(Solve) * nsolve, hipMemcpyHostToDevice, st));
-  HIPCHK(h, hipStreamSynchronize(st));   // the lists above are host memory of this call
-  const int rc = plan_af(h, st);
-  if (rc) return rc;
-  if (h->general) return plan_general(h);
-  return plan_self(h, st);
+  HIPCHK(h, hipMemcpyAsync(dev, list.data(), sizeof(int4) * list.size(), hipMemcpyHostToDevice, st));
+  return CSADV_OK;
 }
 
 }  // namespace
@@ -1127,6 +1086,7 @@ int csadv_create(const csadv_solve_desc *solves, int32_t nsolve, int32_t tile, c
   if ((e = hipMalloc(&h->dev, sizeof(Solve) * nsolve)) != hipSuccess ||
       (e = hipMalloc(&h->qsets, sizeof(FieldSet) * nsolve)) != hipSuccess ||
       (e = hipMalloc(&h->wsets, sizeof(FieldSet) * nsolve)) != hipSuccess ||
+      (e = hipMalloc(&h->plan, sizeof(PlanWords) * nsolve)) != hipSuccess ||
       (e = hipMalloc(&h->fold, sizeof(double) * 2 * maxtr * nsolve)) != hipSuccess ||
       (e = hipMalloc(&h->red, sizeof(double) * diag_scratch_words(maxtr))) != hipSuccess)
     return fail(h, CSADV_E_HIP, std::string("descriptor allocation: ") + hipGetErrorString(e));
@@ -1173,16 +1133,47 @@ int csadv_update(csadv_t *h, const csadv_solve_desc *solves, int32_t nsolve, voi
     const int rc = check_compatible(solves, nsolve, msg);
     if (rc != CSADV_OK) return fail(h, rc, msg);
   }
-  const int rc = upload_plan(h, st);
+  plan_modes(h);
+  h->mfaf = false;
+  for (int s = 0; s < nsolve; ++s) h->mfaf = h->mfaf || (!h->general && h->desc[s].mf == 2);
+  // workgroup b runs on XCD b % kXcds (the list interleaves one band of row segments per XCD); the
+  // FP32 multi-solve step kernel marches two tracers per item (kStepGroup in csadv_step.hpp)
+  const std::vector<Item> work = work_list(h->host, !h->general && h->dtype == CSADV_F32 && nsolve > 1 ? 2 : 1);
+  std::vector<Item> ww, gw;
+  int rc = upload_list(h, work, h->work, h->nwork, st);
   if (rc) return rc;
+  if (nsolve > 1) {                  // the ghost fill and the winds of a multi-solve handle read their own lists
+    ww = wind_list(h->host, h->nwunsteady);
+    gw = ghost_list(h->host);
+    if ((rc = upload_list(h, ww, h->wwork, h->nwwork, st)) || (rc = upload_list(h, gw, h->gwork, h->ngwork, st)))
+      return rc;
+  }
+  HIPCHK(h, hipMemcpyAsync(h->dev, h->host.data(), sizeof(Solve) * nsolve, hipMemcpyHostToDevice, st));
   HIPCHK(h, hipMemcpyAsync(h->qsets, sets.data(), sizeof(FieldSet) * nsolve, hipMemcpyHostToDevice, st));
-  // steps already completed by each solve (a handle may be built over solves that have run)
-  std::vector<int32_t> ctl(4 * nsolve);
-  for (int s = 0; s < nsolve; ++s)
-    HIPCHK(h, hipMemcpyAsync(ctl.data() + 4 * s, solves[s].ctl, 4 * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+  // what the plan needs from the device, in one copy: the steps already completed by each solve (a
+  // handle may be built over solves that have run), its orientation table, and whether its recipes
+  // are in the order of the self-filling step
+  std::vector<PlanWords> got(nsolve);
+  hipLaunchKernelGGL(k_gather_plan, dim3(nsolve), dim3(BLOCK), 0, st, h->dev, h->plan);
+  if ((rc = plan_self(h, &h->plan->ok, st))) return rc;
+  HIPCHK(h, hipMemcpyAsync(got.data(), h->plan, sizeof(PlanWords) * nsolve, hipMemcpyDeviceToHost, st));
   HIPCHK(h, hipStreamSynchronize(st));
-  for (int s = 0; s < nsolve; ++s) h->done[s] = ctl[4 * s + 1];
-  return CSADV_OK;
+  h->af.assign(nsolve, AfSides{});
+  for (int s = 0; s < nsolve; ++s) {
+    h->done[s] = got[s].ctl[1];
+    if (solves[s].mf != 2) continue;
+    for (int t = 0; t < 24; ++t) h->af[s].side[t] = af_side(got[s].orient + 7 * t, t & 3, solves[s].N);
+  }
+  if (h->self) {
+    h->self = got[0].ok != 0;
+    const Solve &S = h->host[0];
+    h->sides.resize(24);
+    for (int t = 0; t < 24; ++t) {
+      const int32_t *r = got[0].orient + 7 * t;
+      h->sides[t] = {r[0] * (int)S.pstride + r[4] * S.d.ld + r[1], r[5] * S.d.ld + r[2], r[6] * S.d.ld + r[3]};
+    }
+  }
+  return h->general ? plan_general(h) : CSADV_OK;
 }
 
 int csadv_bind_flux_tables(csadv_t *h, void *const *tables, void *stream) {
@@ -1200,7 +1191,10 @@ int csadv_bind_flux_tables(csadv_t *h, void *const *tables, void *stream) {
   for (int s = 0; s < ns; ++s) h->ftab[s] = tables ? tables[s] : nullptr;
   drop_graph(h);   // the kernels of a step change with the binding
   hipStream_t st = (hipStream_t)stream;
-  return upload_plan(h, st);
+  plan_modes(h);
+  HIPCHK(h, hipMemcpyAsync(h->dev, h->host.data(), sizeof(Solve) * ns, hipMemcpyHostToDevice, st));
+  HIPCHK(h, hipStreamSynchronize(st));
+  return CSADV_OK;
 }
 
 int csadv_refresh_winds(csadv_t *h, void *stream) {
@@ -1675,6 +1669,7 @@ void csadv_destroy(csadv_t *h) {
   if (h->wsets) (void)hipFree(h->wsets);
   if (h->red) (void)hipFree(h->red);
   if (h->fold) (void)hipFree(h->fold);
+  if (h->plan) (void)hipFree(h->plan);
   if (h->gp_work) (void)hipFree(h->gp_work);
   for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
   drop_graph(h);

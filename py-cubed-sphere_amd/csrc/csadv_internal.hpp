@@ -13,6 +13,12 @@
 
 using namespace csadv;
 
+// What csadv_update reads back of a solve: its control words, its orientation table, and whether its
+// recipes are in the order of the self-filling step.
+struct PlanWords {
+  int32_t ctl[4], orient[24 * 7], ok;
+};
+
 struct csadv_s {
   std::vector<csadv_solve_desc> desc;
   std::vector<Solve> host;
@@ -44,6 +50,7 @@ struct csadv_s {
   std::vector<SelfSide> sides;    // self: the ghost sources of the 24 panel sides
   std::vector<void *> ftab;       // the bound flux tables, one per solve (null: none)
   double *red = nullptr;          // diagnostics scratch: partials and outputs (diag_scratch_words)
+  PlanWords *plan = nullptr;      // device words of csadv_update, one per solve
   double *fold = nullptr;         // csadv_finalize: [solve][red_tracers][2] totals and offsets
   int red_tracers = 1;            // tracers the diagnostics scratch holds (the largest ntr)
   std::vector<int> done;          // host copy of the steps completed per solve (ctl[1])
