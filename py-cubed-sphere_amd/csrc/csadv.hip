@@ -1082,14 +1082,21 @@ int csadv_create(const csadv_solve_desc *solves, int32_t nsolve, int32_t tile, c
   h->done.assign(nsolve, 0);
   h->ftab.assign(nsolve, nullptr);
   h->red_tracers = maxtr;
-  hipError_t e;
-  if ((e = hipMalloc(&h->dev, sizeof(Solve) * nsolve)) != hipSuccess ||
-      (e = hipMalloc(&h->qsets, sizeof(FieldSet) * nsolve)) != hipSuccess ||
-      (e = hipMalloc(&h->wsets, sizeof(FieldSet) * nsolve)) != hipSuccess ||
-      (e = hipMalloc(&h->plan, sizeof(PlanWords) * nsolve)) != hipSuccess ||
-      (e = hipMalloc(&h->fold, sizeof(double) * 2 * maxtr * nsolve)) != hipSuccess ||
-      (e = hipMalloc(&h->red, sizeof(double) * diag_scratch_words(maxtr))) != hipSuccess)
-    return fail(h, CSADV_E_HIP, std::string("descriptor allocation: ") + hipGetErrorString(e));
+  // the handle's tables in one allocation (a serving loop makes and drops handles all the time)
+  size_t at = 0;
+  const auto part = [&](size_t bytes) { const size_t o = at; at += (bytes + 255) / 256 * 256; return o; };
+  const size_t o_dev = part(sizeof(Solve) * nsolve), o_q = part(sizeof(FieldSet) * nsolve),
+               o_w = part(sizeof(FieldSet) * nsolve), o_plan = part(sizeof(PlanWords) * nsolve),
+               o_fold = part(sizeof(double) * 2 * maxtr * nsolve),
+               o_red = part(sizeof(double) * diag_scratch_words(maxtr));
+  const hipError_t e = hipMalloc(&h->tables, at);
+  if (e != hipSuccess) return fail(h, CSADV_E_HIP, std::string("descriptor allocation: ") + hipGetErrorString(e));
+  h->dev = reinterpret_cast<Solve *>(h->tables + o_dev);
+  h->qsets = reinterpret_cast<FieldSet *>(h->tables + o_q);
+  h->wsets = reinterpret_cast<FieldSet *>(h->tables + o_w);
+  h->plan = reinterpret_cast<PlanWords *>(h->tables + o_plan);
+  h->fold = reinterpret_cast<double *>(h->tables + o_fold);
+  h->red = reinterpret_cast<double *>(h->tables + o_red);
   return csadv_update(h, solves, nsolve, nullptr);
 }
 
@@ -1140,13 +1147,15 @@ int csadv_update(csadv_t *h, const csadv_solve_desc *solves, int32_t nsolve, voi
   // FP32 multi-solve step kernel marches two tracers per item (kStepGroup in csadv_step.hpp)
   const std::vector<Item> work = work_list(h->host, !h->general && h->dtype == CSADV_F32 && nsolve > 1 ? 2 : 1);
   std::vector<Item> ww, gw;
-  int rc = upload_list(h, work, h->work, h->nwork, st);
-  if (rc) return rc;
-  if (nsolve > 1) {                  // the ghost fill and the winds of a multi-solve handle read their own lists
+  int rc;
+  if (nsolve > 1) {                  // the kernels of a handle of one solve compute their items
     ww = wind_list(h->host, h->nwunsteady);
     gw = ghost_list(h->host);
-    if ((rc = upload_list(h, ww, h->wwork, h->nwwork, st)) || (rc = upload_list(h, gw, h->gwork, h->ngwork, st)))
+    if ((rc = upload_list(h, work, h->work, h->nwork, st)) || (rc = upload_list(h, ww, h->wwork, h->nwwork, st)) ||
+        (rc = upload_list(h, gw, h->gwork, h->ngwork, st)))
       return rc;
+  } else {
+    h->nwork = (int)work.size();
   }
   HIPCHK(h, hipMemcpyAsync(h->dev, h->host.data(), sizeof(Solve) * nsolve, hipMemcpyHostToDevice, st));
   HIPCHK(h, hipMemcpyAsync(h->qsets, sets.data(), sizeof(FieldSet) * nsolve, hipMemcpyHostToDevice, st));
@@ -1660,16 +1669,11 @@ const char *csadv_last_error(csadv_t *h) { return h ? h->err.c_str() : "null han
 
 void csadv_destroy(csadv_t *h) {
   if (!h) return;
-  if (h->dev) (void)hipFree(h->dev);
+  if (h->tables) (void)hipFree(h->tables);
   if (h->work) (void)hipFree(h->work);
   if (h->gwork) (void)hipFree(h->gwork);
   if (h->wwork) (void)hipFree(h->wwork);
   if (h->spart) (void)hipFree(h->spart);
-  if (h->qsets) (void)hipFree(h->qsets);
-  if (h->wsets) (void)hipFree(h->wsets);
-  if (h->red) (void)hipFree(h->red);
-  if (h->fold) (void)hipFree(h->fold);
-  if (h->plan) (void)hipFree(h->plan);
   if (h->gp_work) (void)hipFree(h->gp_work);
   for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
   drop_graph(h);

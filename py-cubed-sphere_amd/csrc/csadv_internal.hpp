@@ -22,8 +22,9 @@ struct PlanWords {
 struct csadv_s {
   std::vector<csadv_solve_desc> desc;
   std::vector<Solve> host;
+  char *tables = nullptr;         // one allocation: dev, qsets, wsets, plan, fold, red
   Solve *dev = nullptr;           // device descriptors (caller-visible scratch is not used)
-  int4 *work = nullptr;           // step work items
+  int4 *work = nullptr;           // step work items of a multi-solve handle
   int4 *gwork = nullptr;          // ghost-fill work items of a multi-solve handle (ghost_list)
   int4 *wwork = nullptr;          // wind work items of a multi-solve handle (wind_list)
   FieldSet *qsets = nullptr;      // ghost-fill sets for the tracers
