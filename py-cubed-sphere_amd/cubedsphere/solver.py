@@ -46,6 +46,9 @@ def _host(a):
 # Pinned staging of a device-to-host copy, two buffers of this size at most (from torch's caching
 # host allocator, which hands them out per call and takes them back).
 STAGE_BYTES = 4 << 20
+# Below this a copy straight to pageable memory is the faster: 35 us against 51 at 0.5 MB, 64 and 62
+# at 1 MB, 123 against 84 at 2 MB.
+STAGE_MIN = 1 << 20
 
 
 def to_host(t):
@@ -53,10 +56,12 @@ def to_host(t):
     buffers while the previous ones are copied on: a copy straight to pageable memory took 0.80 ms
     for 14 MB and 13.6 ms for 57 MB, this one 0.35 and 2.3 ms."""
     t = t.contiguous()
+    if t.numel() * t.element_size() < STAGE_MIN:
+        return t.cpu().numpy()
     out = np.empty(tuple(t.shape), dtype=torch.empty(0, dtype=t.dtype).numpy().dtype)
     src, dst = t.view(-1).view(torch.uint8), torch.from_numpy(out.reshape(-1)).view(torch.uint8)
     n, chunk = src.numel(), min(src.numel(), STAGE_BYTES)
-    pieces = [(a, min(n, a + chunk)) for a in range(0, n, max(chunk, 1))]
+    pieces = [(a, min(n, a + chunk)) for a in range(0, n, chunk)]
     stage = [torch.empty(chunk, dtype=torch.uint8, pin_memory=True) for _ in pieces[:2]]
     done = [torch.cuda.Event() for _ in stage]
     stream = torch.cuda.current_stream(t.device)
@@ -71,8 +76,7 @@ def to_host(t):
         done[k & 1].record(stream)
         if k:
             take(k - 1)
-    if pieces:
-        take(len(pieces) - 1)
+    take(len(pieces) - 1)
     return out
 
 
