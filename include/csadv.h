@@ -150,7 +150,8 @@ int csadv_wind_init(csadv_t *h, void *stream);
  * before csadv_wind_init, which fills the tables; the steps of a time-dependent solve refresh
  * them.  A filled table may be bound to any later handle over the same solve (same dt, dx, options
  * and winds) without another csadv_wind_init.  A solve with RK1 and a one-field time-dependent wind
- * uses none (the step forms its winds).  csadv_update keeps the binding.  No counterpart in the reference. */
+ * uses none (the step forms its winds).  csadv_update keeps the binding of a solve whose
+ * step, grid, options and wind buffers it leaves as they were and drops it otherwise.  No counterpart in the reference. */
 int csadv_flux_table_bytes(int32_t N, int32_t split, int64_t *bytes);
 int csadv_bind_flux_tables(csadv_t *h, void *const *tables, void *stream);
 

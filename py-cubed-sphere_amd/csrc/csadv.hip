@@ -1100,6 +1100,14 @@ int csadv_create(const csadv_solve_desc *solves, int32_t nsolve, int32_t tile, c
   return csadv_update(h, solves, nsolve, nullptr);
 }
 
+// Whether a flux table filled for `a` holds the weights of `b`.
+static bool same_weights(const csadv_solve_desc &a, const csadv_solve_desc &b) {
+  return a.N == b.N && a.dtype == b.dtype && a.ld == b.ld && a.ldu == b.ldu && a.recon == b.recon && a.dp == b.dp &&
+         a.split == b.split && a.et == b.et && a.mt == b.mt && a.unsteady == b.unsteady && a.dt == b.dt &&
+         a.dx == b.dx && a.dy == b.dy && a.uavg == b.uavg && a.vavg == b.vavg && a.usgn == b.usgn &&
+         a.vsgn == b.vsgn && a.gc == b.gc && a.gu == b.gu && a.gv == b.gv && a.rgc == b.rgc;
+}
+
 int csadv_update(csadv_t *h, const csadv_solve_desc *solves, int32_t nsolve, void *stream) {
   if (!h) return CSADV_E_ARG;
   if (!solves || nsolve != (int)h->desc.size()) return fail(h, CSADV_E_ARG, "solve count mismatch");
@@ -1115,6 +1123,7 @@ int csadv_update(csadv_t *h, const csadv_solve_desc *solves, int32_t nsolve, voi
       msg = "ntr grew past the handle's diagnostics scratch (create a new handle)";
     }
     if (rc != CSADV_OK) return fail(h, rc, "solve " + std::to_string(s) + ": " + msg);
+    if (!same_weights(h->desc[s], solves[s])) h->ftab[s] = nullptr;   // the step forms the new ones
     h->desc[s] = solves[s];
     const Solve S = derive(solves[s], h->tile);
     h->host.push_back(S);

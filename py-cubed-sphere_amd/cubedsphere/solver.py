@@ -305,6 +305,7 @@ class Advection:
         use = self.case.steady and self.dtype == "f64" and not general
         nbytes = flux_table_bytes(N, self.opts["split"]) if use else 0
         self.flux_table = torch.zeros(nbytes, device=dev, dtype=torch.uint8) if nbytes else None
+        self.flux_key = None          # the step and options the table was filled for
         if not general and self.opts["mf"] == 2:
             self.work = torch.zeros(ntr * 24 * N, device=dev, dtype=td)
 
@@ -312,12 +313,18 @@ class Advection:
     def bind_flux_tables(lib, handle, members, stream, fill=False):
         """Hand the members' flux tables to their handle (csadv_bind_flux_tables).  The members step
         with them only where all of them together stay in cache (weights formed in the step have the
-        same bits); ``fill``: bound to be filled by csadv_wind_init."""
-        total = sum(m.flux_table.numel() for m in members if m.flux_table is not None)
+        same bits); ``fill``: bound to be filled by csadv_wind_init, for the step and the options the
+        members have now.  A table of another step or other options is left out."""
+        use = []
+        for m in members:
+            key = (m.dt, tuple(sorted(m.opts.items())))
+            if m.flux_table is not None and fill:
+                m.flux_key = key if m.flux_table.numel() == flux_table_bytes(m.grid.N, m.opts["split"]) else None
+            use.append(m.flux_table if m.flux_table is not None and m.flux_key == key else None)
+        total = sum(t.numel() for t in use if t is not None)
         if total == 0 or (total > FLUX_TABLE_MAX and not fill):
             return
-        tabs = (ctypes.c_void_p * len(members))(*[m.flux_table.data_ptr() if m.flux_table is not None else None
-                                                  for m in members])
+        tabs = (ctypes.c_void_p * len(members))(*[None if t is None else t.data_ptr() for t in use])
         _lib.check(lib.csadv_bind_flux_tables(handle, tabs, stream), handle, "csadv_bind_flux_tables")
 
     def device_bytes(self):
@@ -372,7 +379,7 @@ class Advection:
         rc = self.lib.csadv_create(ctypes.byref(d), 1, self.tile, ctypes.byref(h))
         self.handle = h
         _lib.check(rc, h, "csadv_create")
-        self.bind_flux_tables(self.lib, h, [self], self._stream())
+        self.bind_flux_tables(self.lib, h, [self], self._stream(), fill=True)
         _lib.check(self.lib.csadv_wind_init(h, self._stream()), h, "csadv_wind_init")
         return self
 

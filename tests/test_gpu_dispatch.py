@@ -69,6 +69,28 @@ def test_flux_tables_have_the_bits_of_formed_weights(N, opts, monkeypatch):
     _same(_run(N, _steady(2), [5], **opts), with_table)
 
 
+@pytest.mark.parametrize("change", ["dt", "recon", "opsplit"])
+def test_flux_tables_of_another_step_are_left_out(change, monkeypatch):
+    from cubedsphere.solver import Advection
+
+    def run():
+        sol = Advection(21, _steady(1), 0.01, device="cuda:0", max_steps=8).init_vars_adv()
+        sol.step(3)
+        if change == "dt":
+            sol.dt *= 0.5
+        else:
+            sol.opts["recon" if change == "recon" else "split"] = 2
+        sol.refresh()
+        sol.step(3)
+        out = sol.full_state()
+        sol.close()
+        return out
+
+    with_table = run()
+    monkeypatch.setattr(Advection, "bind_flux_tables", staticmethod(lambda *a, **k: None))
+    assert np.array_equal(with_table, run())
+
+
 @pytest.mark.parametrize("dp,dtype", [(1, "f64"), (2, "f64"), (2, "f32")])
 def test_steady_and_unsteady_solves_in_one_handle(dp, dtype):
     from cubedsphere.batch import Batch, make_members
