@@ -5,17 +5,21 @@
 //                                     used by csadv_ghost_fill and for the wind basis
 //   k_ghost                           per-step ghost fill of the 3 layers a step reads, from
 //                                     flattened recipes, plus the MF-PR sum of the last step
-//   k_step<T,RECON,RK2,SPLIT,WIND>    the step: both directional passes of the split, PPM edges,
+//   k_step<T,RECON,MODE,SPLIT>        the step: both directional passes of the split, PPM edges,
 //                                     upwind fluxes, update and the mass-fixer partial sums of one
 //                                     (solve, panel, tracer, column strip, row segment) per
 //                                     wavefront (src/discrete_operators.py:18-101, src/flux.py,
 //                                     src/reconstruction_1d.py); k_step1 is the same for a handle
-//                                     of one solve, whose descriptor is a kernel argument
-//   gp::k_gp_* (csadv_general.hpp)    the general step (ET-S72, ET-PL07): one kernel per
-//                                     stage of src/discrete_operators.py:18-101
+//                                     of one solve, whose descriptor is a kernel argument;
+//                                     k_step_self fills its own ghosts (small solves), k_advance
+//                                     moves the step counter after a sequence of them
+//   k_af_fix                          MF-AF's averages at the boundary cells (fused step)
+//   gp::k_gp_* (csadv_general.hpp)    the general step (ET-S72, ET-PL07): two marched passes and
+//                                     the mass fixers of src/discrete_operators.py:18-101
 //   k_wind_e2c / k_wind_c2e           duo-grid vector ghost fill (src/interpolation.py:347-532)
 //   k_wind_avg                        time-averaged winds (src/averaged_velocity.py:14-62)
 //   k_settle, k_fold_values / k_finalize, k_diag / k_diag_final   state read-out and diagnostics
+//   k_check_recipes, k_gather_plan    what building a handle needs from the device
 // The fused step kernel lives in csadv_step.hpp (instantiated by step_<dtype>_r<recon>.hip), the
 // general step in csadv_general.hpp (general_<dtype>_s<split>.hip), the host-side planning in
 // csadv_plan.cpp.
@@ -612,7 +616,7 @@ constexpr int kMaxBasis = 8;
 template <int KB>
 __device__ __forceinline__ double wind_comb(const double *W, int64_t bs, const double *s, int K) {
   if constexpr (KB == 1) {
-    return wind_of_basis(s[0], W[0]);   // the same bits as the step's own (WIND)
+    return wind_of_basis(s[0], W[0]);   // the same bits as the step's own (kWind)
   } else {
     double acc = 0.0;
 #pragma unroll
