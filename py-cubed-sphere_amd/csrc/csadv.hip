@@ -157,8 +157,9 @@ __device__ double partial_sum(const double *P, int n, double *red) {
 }
 
 // blk: the block of BLOCK ghost cells, or -1 for the tracer's correction-total block; tr: tracer.
-template <typename T>
-__device__ __forceinline__ void ghost_cells(const Solve &S, double *red, int blk, int tr) {
+// PAIR: the cells of tracer tr + 1 as well where `two` is set, by the same recipes.
+template <typename T, bool PAIR>
+__device__ __forceinline__ void ghost_cells(const Solve &S, double *red, int blk, int tr, bool two) {
   const csadv_solve_desc &D = S.d;
   // Every descriptor field of this kernel is requested up front: the empty asm below takes them
   // all, so their scalar loads are issued together before the first branch (one round trip,
@@ -235,19 +236,28 @@ __device__ __forceinline__ void ghost_cells(const Solve &S, double *red, int blk
     return;
   }
   T *Qt = reinterpret_cast<T *>((steps & 1) ? q1 : q0) + tr * tstride;
-  double acc = 0.0;                         // in recipe order
-  if (active) {
+  if (active) {                             // sums in recipe order
     if (strip) {
       const T v0 = Qt[s16[0]], v1 = Qt[s16[1]], v2 = Qt[s16[2]], v3 = Qt[s16[3]];
-      acc = strip_sum((double)v0, (double)v1, (double)v2, (double)v3, w16[0], w16[1], w16[2], w16[3]);
+      if (PAIR && two) {                    // both tracers' sources in flight together
+        T *Qn = Qt + tstride;
+        const T n0 = Qn[s16[0]], n1 = Qn[s16[1]], n2 = Qn[s16[2]], n3 = Qn[s16[3]];
+        Qn[tgt] = (T)strip_sum((double)n0, (double)n1, (double)n2, (double)n3, w16[0], w16[1], w16[2], w16[3]);
+      }
+      Qt[tgt] = (T)strip_sum((double)v0, (double)v1, (double)v2, (double)v3, w16[0], w16[1], w16[2], w16[3]);
     } else {
-      T v[16];
+      // (one after another: the corners are few, and their 32 sources would cost the strips' residency)
+#pragma unroll 1
+      for (int t = PAIR && two ? 2 : 1; t > 0; --t, Qt += tstride) {
+        T v[16];
+        double acc = 0.0;
 #pragma unroll
-      for (int l = 0; l < 16; ++l) v[l] = Qt[s16[l]];
+        for (int l = 0; l < 16; ++l) v[l] = Qt[s16[l]];
 #pragma unroll
-      for (int l = 0; l < 16; ++l) acc = fma((double)v[l], w16[l], acc);
+        for (int l = 0; l < 16; ++l) acc = fma((double)v[l], w16[l], acc);
+        Qt[tgt] = (T)acc;
+      }
     }
-    Qt[tgt] = (T)acc;
   }
   if (lead) ctl[2] = steps;
 }
@@ -279,12 +289,12 @@ __device__ __forceinline__ double settled_total(const Solve &S, int tr) {
   return corr_total(D.dt, D.a2, c0, c1, sum, pending, steps);
 }
 
-// A handle of several solves: workgroup b takes item b of the ghost work list (ghost_list).
+// A handle of several solves: workgroup b takes item b of the ghost work list (ghost_pairs).
 template <typename T>
 __global__ __launch_bounds__(BLOCK) void k_ghost(const Solve *solves, const int4 *gwork) {
   __shared__ double red[BLOCK];
   const int4 it = gwork[blockIdx.x];
-  ghost_cells<T>(solves[it.x], red, it.z, it.y);
+  ghost_cells<T, true>(solves[it.x], red, it.z, it.y, it.w != 0);
 }
 
 // A handle of one solve: the descriptor travels in the kernel arguments.
@@ -292,7 +302,7 @@ template <typename T>
 __global__ __launch_bounds__(BLOCK) void k_ghost1(const Solve one) {
   __shared__ double red[BLOCK];
   // grid (cell blocks + 1, 1, tracers): the last block of each layer is the correction total's
-  ghost_cells<T>(one, red, blockIdx.x == gridDim.x - 1 ? -1 : (int)blockIdx.x, (int)blockIdx.z);
+  ghost_cells<T, false>(one, red, blockIdx.x == gridDim.x - 1 ? -1 : (int)blockIdx.x, (int)blockIdx.z, false);
 }
 
 // csadv_finalize folds the correction totals (interior) and the FP32 state offsets (every cell: a
@@ -1163,7 +1173,7 @@ int csadv_update(csadv_t *h, const csadv_solve_desc *solves, int32_t nsolve, voi
   int rc;
   if (nsolve > 1) {                  // the kernels of a handle of one solve compute their items
     ww = wind_list(h->host, h->nwunsteady);
-    gw = ghost_list(h->host);
+    gw = ghost_pairs(ghost_list(h->host), h->host);
     if ((rc = upload_list(h, work, h->work, h->nwork, st)) || (rc = upload_list(h, ww, h->wwork, h->nwwork, st)) ||
         (rc = upload_list(h, gw, h->gwork, h->ngwork, st)))
       return rc;

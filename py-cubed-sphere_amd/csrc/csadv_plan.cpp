@@ -135,6 +135,15 @@ std::vector<Item> ghost_list(const std::vector<Solve> &solves) {
   return g;
 }
 
+std::vector<Item> ghost_pairs(const std::vector<Item> &list, const std::vector<Solve> &solves) {
+  std::vector<Item> g;
+  for (const Item &it : list) {
+    if (it.z >= 0 && it.y % 2 != 0) continue;
+    g.push_back(Item{it.x, it.y, it.z, it.z >= 0 && it.y + 1 < solves[it.x].d.ntr ? 1 : 0});
+  }
+  return g;
+}
+
 std::vector<Item> wind_list(const std::vector<Solve> &solves, int &unsteady) {
   std::vector<Item> w;
   unsteady = 0;
